@@ -1,0 +1,161 @@
+"""What this library is timed on: GEMMs as user programs call them, through ``Loader.gemm``.
+
+A case is one of two kinds.  ``gemm``: one call, C = A * B, possibly over a strided batch.
+``linear``: the three products of a training step of a linear layer (forward, gradient of
+the input, gradient of the weight), which between them use three of the four pairs of
+operand layouts.  Sizes are the library's own benchmark and test configurations (squares,
+transformer projections, decode-like skinny shapes, ragged and long-K shapes, strided
+batches); ``draw`` spreads over the same ranges.
+"""
+import math
+
+import torch
+
+import rocm_wmma_gemm_amd as R
+
+DTYPES = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+PAIRS = (("f16", "f16"), ("f16", "f32"), ("bf16", "bf16"), ("bf16", "f32"))  # (A and B, C)
+MOST_FLOPS = 2.0 * 8192 ** 3  # no drawn case costs more than the largest listed one
+
+
+def _gemm(name, m, n, k, ab, c, layouts, batch=1):
+    """layouts: of A, B and C in this order, r = row-major, c = column-major."""
+    return {"name": name, "kind": "gemm", "m": m, "n": n, "k": k, "ab": ab, "c": c, "layouts": layouts,
+            "batch": batch}
+
+
+def _linear(name, tokens, features_out, features_in, ab, c):
+    return {"name": name, "kind": "linear", "m": tokens, "n": features_out, "k": features_in, "ab": ab, "c": c}
+
+
+def listed():
+    return [
+        # the smallest problem of the reference harness: one call's latency and host cost
+        _gemm("small_256_f16", 256, 256, 256, "f16", "f16", "rcr"),
+        # a small product that is no whole number of tiles (edge-tile sweep of the benchmark)
+        _gemm("small_1000_bf16", 1000, 1000, 1000, "bf16", "bf16", "crr"),
+        # a strided batch of small products (attention heads, experts)
+        _gemm("batch_64x512_f16", 512, 512, 512, "f16", "f16", "rrr", batch=64),
+        # decode: 16 sequences against a square weight that has to come from memory
+        _gemm("decode_16x8192x8192_f16_f32", 16, 8192, 8192, "f16", "f32", "rcr"),
+        # decode with a number of sequences that no table holds, weights stored K by N
+        _gemm("decode_37x4096x14336_bf16", 37, 4096, 14336, "bf16", "bf16", "rrr"),
+        # a large decode batch: between bandwidth and matrix cores
+        _gemm("decode_128x8192x8192_f16_f32", 128, 8192, 8192, "f16", "f32", "rcr"),
+        # prefill of one prompt (an odd number of tokens) against the largest weight in the tables
+        _gemm("prefill_777x28672x8192_bf16", 777, 28672, 8192, "bf16", "bf16", "rcr"),
+        # training: forward and backward of a projection
+        _linear("linear_4096x5120x5120_bf16", 4096, 5120, 5120, "bf16", "bf16"),
+        # the two headline squares
+        _gemm("square_4096_f16", 4096, 4096, 4096, "f16", "f16", "rcr"),
+        _gemm("square_8192_bf16_f32", 8192, 8192, 8192, "bf16", "f32", "rcr"),
+        # odd in every extent: no row of an operand is aligned
+        _gemm("ragged_4095x5121x3001_bf16", 4095, 5121, 3001, "bf16", "bf16", "rcr"),
+        # a long sum into a small C (a weight gradient over many tokens), mixed layouts
+        _gemm("longk_1024x1024x65536_bf16", 1024, 1024, 65536, "bf16", "bf16", "rrr"),
+    ]
+
+
+def _spread(rng, low, high, grain=1):
+    """A size between low and high, spread over its logarithm, a multiple of grain."""
+    x = math.exp(rng.uniform(math.log(low), math.log(high)))
+    return max(grain, int(round(x / grain)) * grain)
+
+
+def draw(rng):
+    ab, c = PAIRS[rng.randrange(4)]
+    layouts = "".join(rng.choice("rc") for _ in range(3))
+    # most programs keep features on multiples of 64; some only on 8; a few not at all
+    grain = rng.choice((64, 64, 64, 8, 8, 1))
+    kind = rng.randrange(6)
+    batch = 1
+    if kind == 0:  # small, alone or in a batch
+        m, n, k = (_spread(rng, 32, 1024, grain) for _ in range(3))
+        batch = rng.choice((1, 1, _spread(rng, 2, 128)))
+    elif kind == 1:  # decode: any number of rows against a weight
+        m, n, k = _spread(rng, 1, 128), _spread(rng, 1024, 28672, grain), _spread(rng, 1024, 28672, grain)
+        layouts = "r" + layouts[1] + "r"
+    elif kind == 2:  # prefill: any number of tokens against a weight
+        m, n, k = _spread(rng, 129, 4096), _spread(rng, 1024, 16384, grain), _spread(rng, 1024, 16384, grain)
+        layouts = "r" + layouts[1] + "r"
+    elif kind == 3:  # squares and rectangles
+        m, n, k = (_spread(rng, 512, 8192, grain) for _ in range(3))
+    elif kind == 4:  # a long sum into a small C
+        m, n, k = _spread(rng, 256, 2048, grain), _spread(rng, 256, 2048, grain), _spread(rng, 8192, 65536, grain)
+    else:  # training step of a linear layer
+        m, n, k = _spread(rng, 512, 8192, 8), _spread(rng, 512, 8192, grain), _spread(rng, 512, 8192, grain)
+        while 6.0 * m * n * k > MOST_FLOPS:
+            m = max(8, m // 16 * 8)
+        case = _linear("", m, n, k, ab, c)
+        del case["name"]
+        return case
+    while 2.0 * m * n * k * batch > MOST_FLOPS:
+        k = max(8, k // 16 * 8)
+    case = _gemm("", m, n, k, ab, c, layouts, batch)
+    del case["name"]
+    return case
+
+
+def _values(generator, count, dtype):
+    """bf16: normal(0, 1); f16: uniform on [-1, 1] (the benchmark's distributions)."""
+    x = torch.empty(count, dtype=dtype, device="cuda")
+    if dtype is torch.bfloat16:
+        return x.normal_(generator=generator)
+    return x.uniform_(-1.0, 1.0, generator=generator)
+
+
+_CODE = {"r": R.row_major, "c": R.col_major}
+
+
+def prepare(case, seed):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    m, n, k = case["m"], case["n"], case["k"]
+    ab, c = DTYPES[case["ab"]], DTYPES[case["c"]]
+    state = {"loader": R.Loader(), "kind": case["kind"], "m": m, "n": n, "k": k}
+    if case["kind"] == "linear":
+        state["x"] = _values(g, m * k, ab)
+        state["w"] = _values(g, n * k, ab)
+        state["dy"] = _values(g, m * n, ab)
+        state["y"] = torch.empty(m * n, dtype=c, device="cuda")
+        state["dx"] = torch.empty(m * k, dtype=c, device="cuda")
+        state["dw"] = torch.empty(n * k, dtype=c, device="cuda")
+        return state
+    batch = case["batch"]
+    state["a"] = _values(g, m * k * batch, ab)
+    state["b"] = _values(g, k * n * batch, ab)
+    state["out"] = torch.empty(m * n * batch, dtype=c, device="cuda")
+    state["batch"] = batch
+    state["la"], state["lb"], state["lc"] = (_CODE[x] for x in case["layouts"])
+    return state
+
+
+def run(state):
+    gemm, m, n, k = state["loader"].gemm, state["m"], state["n"], state["k"]
+    if state["kind"] == "linear":
+        r, c = R.row_major, R.col_major
+        # X is tokens x in, W is out x in, both row-major: Y = X W^T, dX = dY W, dW = dY^T X
+        gemm(state["y"], state["x"], state["w"], m, n, k, r, r, c)
+        gemm(state["dx"], state["dy"], state["w"], m, k, n, r, r, r)
+        gemm(state["dw"], state["dy"], state["x"], n, k, m, r, c, r)
+        return {"y": state["y"], "dx": state["dx"], "dw": state["dw"]}
+    gemm(state["out"], state["a"], state["b"], m, n, k, state["lc"], state["la"], state["lb"], state["batch"])
+    return state["out"]
+
+
+def work(case):
+    m, n, k = case["m"], case["n"], case["k"]
+    size = 4 if case["c"] == "f32" else 2
+    if case["kind"] == "linear":
+        elements = m * k + n * k + m * n
+        return {"bytes": 2 * elements + size * elements, "flops": 6.0 * m * n * k}
+    batch = case["batch"]
+    return {"bytes": batch * (2 * (m * k + k * n) + size * m * n), "flops": 2.0 * batch * m * n * k}
+
+
+def tolerance(case):
+    # Against the same product in float64 every case shows the rounding of C's type alone:
+    # rel 2.1e-4 in f16, 1.66e-3 in bf16 (max: half a unit in the last place, 4.9e-4 and
+    # 3.9e-3); f32 out up to 1.4e-6 (max 8.5e-6) at K = 46741.  Four times that.
+    return {"f16": {"rel": 8e-4, "max": 2e-3}, "bf16": {"rel": 6.6e-3, "max": 1.6e-2},
+            "f32": {"rel": 6e-6, "max": 3.5e-5}}[case["c"]]
