@@ -159,3 +159,25 @@ def tolerance(case):
     # 3.9e-3); f32 out up to 1.4e-6 (max 8.5e-6) at K = 46741.  Four times that.
     return {"f16": {"rel": 8e-4, "max": 2e-3}, "bf16": {"rel": 6.6e-3, "max": 1.6e-2},
             "f32": {"rel": 6e-6, "max": 3.5e-5}}[case["c"]]
+
+
+def exact(case, seed):
+    """What run() returns for these inputs, in float64: plain matrix products, no code of this library."""
+    s = prepare(case, seed)
+    m, n, k = case["m"], case["n"], case["k"]
+    if case["kind"] == "linear":
+        x, w, dy = (s[key].double().view(shape) for key, shape in (("x", (m, k)), ("w", (n, k)), ("dy", (m, n))))
+        return {"y": (x @ w.t()).flatten(), "dx": (dy @ w).flatten(), "dw": (dy.t() @ x).flatten()}
+
+    def matrix(flat, rows, columns, layout):
+        if layout == "r":
+            return flat.view(case["batch"], rows, columns)
+        return flat.view(case["batch"], columns, rows).transpose(1, 2)
+
+    a = matrix(s["a"].double(), m, k, case["layouts"][0])
+    b = matrix(s["b"].double(), k, n, case["layouts"][1])
+    out = torch.empty(m * n * case["batch"], dtype=torch.float64, device="cuda")
+    c = matrix(out, m, n, case["layouts"][2])
+    for i in range(case["batch"]):
+        c[i] = a[i] @ b[i]
+    return out
