@@ -588,7 +588,7 @@ struct direct_gemm
         {
             batch = blockIdx.y;
             w     = decode_block(args);
-            t     = map_tile(w.tile_id, args.grid_m, args.grid_n, args.group);
+            t     = tile_of(args, w);
         }
         const int slice = w.slice;
         const int row0 = t.m * BM;

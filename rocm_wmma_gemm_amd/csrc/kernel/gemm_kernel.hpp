@@ -109,24 +109,44 @@ struct gemm_args
                                // in that cache (16 x 8192 x 8192 20.6 us, 29 with the hint).
 };
 
-// What one workgroup works on.  blockIdx.x enumerates the whole tiles first, then
-// (slice, split tile) pairs, slices outermost.
+// What one workgroup works on.  Ids enumerate the whole tiles first, then (slice, split
+// tile) pairs, slices outermost.
 struct block_work
 {
-    int tile_id; // position in the tile walk (see map_tile)
-    int slice, slices; // K slice of this workgroup and how many the tile has (1 = whole K)
+    int  tile_id; // position in the tile walk
+    int  slice, slices; // K slice of this workgroup and how many the tile has (1 = whole K)
+    bool walk_order; // tile_id counts along the walk already (see tile_of), else it is dealt by XCD
 };
 
+// Where every tile is split, the ids of the launch are renumbered as a whole, so that an XCD
+// owns a contiguous run of (slice, tile) pairs, a slice or two of K over all tiles.  Its L2 then
+// fetches its part of A and B once; with the tiles of every slice dealt over the XCDs,
+// as whole tiles are, each of the 8 L2s fetched nearly all of both operands, and the
+// fabric was the bound (704 x 896 x 12096 in 16 slices
+// 47.7 -> 44.5 us, 2048 x 1024 x 32768 in 8 145.7 -> 137.3, operands from HBM; a few slices of many
+// tiles gain nothing and lose nothing).
 __device__ __forceinline__ block_work decode_block(const gemm_args& args, int b)
 {
     if(b < args.tail_begin || args.k_slices == 1)
     {
-        return {b, 0, 1};
+        return {b, 0, 1, false};
     }
     const int split_tiles = args.grid_m * args.grid_n - args.tail_begin;
-    const int r           = b - args.tail_begin;
-    const int slice       = r / split_tiles;
-    return {args.tail_begin + (r - slice * split_tiles), slice, args.k_slices};
+    if(args.tail_begin == 0)
+    {
+        const int item  = xcd_remap(b, split_tiles * args.k_slices);
+        const int slice = item / split_tiles;
+        return {item - slice * split_tiles, slice, args.k_slices, true};
+    }
+    const int r     = b - args.tail_begin;
+    const int slice = r / split_tiles;
+    return {args.tail_begin + (r - slice * split_tiles), slice, args.k_slices, false};
+}
+
+__device__ __forceinline__ tile_coord tile_of(const gemm_args& args, const block_work& w)
+{
+    return banded_tile(w.walk_order ? w.tile_id : xcd_remap(w.tile_id, args.grid_m * args.grid_n), args.grid_m,
+                       args.grid_n, args.group);
 }
 
 __device__ __forceinline__ block_work decode_block(const gemm_args& args)
@@ -502,7 +522,7 @@ struct staged_gemm
         // blockIdx.x enumerates tiles and K slices; blockIdx.y the batch entry.
         const block_work w = decode_block(args);
         const int slice    = w.slice;
-        const tile_coord t = map_tile(w.tile_id, args.grid_m, args.grid_n, args.group);
+        const tile_coord t = tile_of(args, w);
         const int row0 = t.m * BM;
         const int col0 = t.n * BN;
 

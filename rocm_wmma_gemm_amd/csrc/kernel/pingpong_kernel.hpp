@@ -116,7 +116,7 @@ struct pingpong_gemm
 
         const block_work w = decode_block(args);
         const int slice    = w.slice;
-        const tile_coord t = map_tile(w.tile_id, args.grid_m, args.grid_n, args.group);
+        const tile_coord t = tile_of(args, w);
         const int row0 = t.m * BM;
         const int col0 = t.n * BN;
 

@@ -716,7 +716,7 @@ struct solo_gemm
             const block_work w = decode_block(args, item - x.batch * args.blocks_per_batch);
             const tile_coord t = args.batch_by_xcd
                                      ? banded_tile(w.tile_id, args.grid_m, args.grid_n, args.group)
-                                     : map_tile(w.tile_id, args.grid_m, args.grid_n, args.group);
+                                     : tile_of(args, w);
             x.row0             = t.m * BM;
             x.col0             = t.n * BN;
             const int steps_per = (k_steps_total + w.slices - 1) / w.slices;
