@@ -1002,7 +1002,8 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
         if(split_k > 1 && tail_begin == 0)
         {
             const long long plane  = static_cast<long long>(p.M) * static_cast<long long>(p.N);
-            const int       blocks = static_cast<int>(std::min<long long>((plane + 255) / 256, 4096));
+            // (four elements a thread; a ragged plane takes more turns)
+            const int       blocks = static_cast<int>(std::min<long long>((plane + 1023) / 1024, 4096));
             enqueue(&device::reduce_partials<OutT>, dim3(blocks, static_cast<unsigned>(nb)), dim3(256), stream,
                     static_cast<OutT*>(args.C), partials, plane, split_k, args.batch_stride_c);
         }

@@ -665,7 +665,67 @@ __global__ void __launch_bounds__(Impl::THREADS) gemm_entry(const gemm_args args
 }
 
 // Sums the k_slices fp32 partial planes of split-K in ascending slice order and
-// writes C (row-major M x N per batch entry) in its own element type.
+// writes C (row-major M x N per batch entry) in its own element type.  A plane is a few
+// MB that lies in the caches: the bound is how many loads are on their way, so a thread takes 4
+// elements and has the loads of 8 planes out before it adds the first (704 x 896 in 16
+// planes: the call 44.5 -> 41.3 us; 960 x 256 in 32: 37.2 -> 33.6).  A
+// plane or C that is not 4 elements wide throughout goes one element a thread.
+template<class OutT, int WIDTH>
+__device__ __forceinline__ void reduce_planes(OutT* __restrict__ out,
+                                              const float* __restrict__ P,
+                                              long long plane,
+                                              int       k_slices)
+{
+    typedef float in_t __attribute__((ext_vector_type(WIDTH)));
+    typedef OutT  out_t __attribute__((ext_vector_type(WIDTH)));
+    constexpr int AHEAD = 8;
+    for(long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * WIDTH; i < plane;
+        i += (long long)gridDim.x * blockDim.x * WIDTH)
+    {
+        in_t s = in_t(0.0f);
+        int  k = 0;
+        for(; k + AHEAD <= k_slices; k += AHEAD)
+        {
+            in_t v[AHEAD];
+#pragma unroll
+            for(int u = 0; u < AHEAD; ++u)
+            {
+                v[u] = *reinterpret_cast<const in_t*>(P + (k + u) * plane + i);
+            }
+#pragma unroll
+            for(int u = 0; u < AHEAD; ++u)
+            {
+                s += v[u];
+            }
+        }
+        // what is left, up to AHEAD - 1 planes: the planes past the last are not read
+        in_t v[AHEAD - 1];
+#pragma unroll
+        for(int u = 0; u < AHEAD - 1; ++u)
+        {
+            if(k + u < k_slices)
+            {
+                v[u] = *reinterpret_cast<const in_t*>(P + (k + u) * plane + i);
+            }
+        }
+#pragma unroll
+        for(int u = 0; u < AHEAD - 1; ++u)
+        {
+            if(k + u < k_slices)
+            {
+                s += v[u];
+            }
+        }
+        out_t o;
+#pragma unroll
+        for(int x = 0; x < WIDTH; ++x)
+        {
+            o[x] = to_out<OutT>(s[x]);
+        }
+        *reinterpret_cast<out_t*>(out + i) = o;
+    }
+}
+
 template<class OutT>
 __global__ void __launch_bounds__(256) reduce_partials(OutT* __restrict__ C,
                                                        const float* __restrict__ partials,
@@ -676,15 +736,13 @@ __global__ void __launch_bounds__(256) reduce_partials(OutT* __restrict__ C,
     const long long batch = blockIdx.y;
     const float*    P     = partials + batch * k_slices * plane;
     OutT*           out   = C + batch * batch_stride_c;
-    for(long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < plane;
-        i += (long long)gridDim.x * blockDim.x)
+    if(plane % 4 == 0 && (unsigned long long)out % (4 * sizeof(OutT)) == 0)
     {
-        float s = 0.0f;
-        for(int k = 0; k < k_slices; ++k)
-        {
-            s += P[k * plane + i];
-        }
-        out[i] = to_out<OutT>(s);
+        reduce_planes<OutT, 4>(out, P, plane, k_slices);
+    }
+    else
+    {
+        reduce_planes<OutT, 1>(out, P, plane, k_slices);
     }
 }
 
