@@ -314,6 +314,20 @@ struct operand_stage
             {
                 int row, chunk;
                 chunk_of(i, tid, row, chunk);
+                if constexpr(KMAJOR)
+                {
+                    // A chunk that the row holds whole is one 16-byte load at whatever
+                    // address it starts on (an ordinary unaligned load to the compiler); only
+                    // the chunk that K cuts goes element by element.  Eight loads of 2 bytes
+                    // for each bound the skinny shapes with an odd K (16 x 8192 x
+                    // 8191: 125 -> 61 us, with the tile that the dispatcher picks for them).
+                    typedef u32x4 any_u32x4 __attribute__((aligned(2)));
+                    if(row < rows_left && chunk * 8 + 8 <= k_left)
+                    {
+                        regs[i] = *reinterpret_cast<const any_u32x4*>(base + row * stride_row + chunk * 8);
+                        continue;
+                    }
+                }
                 unsigned short e[8];
 #pragma unroll
                 for(int j = 0; j < 8; ++j)
