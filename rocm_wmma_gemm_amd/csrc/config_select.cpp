@@ -156,6 +156,9 @@ bool step_cost(const model_variant& v, double* step_us, double* item_us)
     return false;
 }
 
+// the general kernel's smallest square tile, 64 x 64 x 64
+constexpr int small_general_variant = 34;
+
 size_t ceil_div(size_t a, size_t b)
 {
     return (a + b - 1) / b;
@@ -171,8 +174,12 @@ size_t ceil_div(size_t a, size_t b)
 // with the second less than half full) and ran at 0.7 of the 196 tiles of 256 x 256.
 // On the 208 tuned entries the model can serve, its pick is on average 2.7 % slower than
 // the tuner's, 25 % at worst.
-bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch,
-                size_t cus_of_device)
+//
+// `any_rows`: also for extents whose rows do not start on 16 bytes (see model_plan_any_rows).
+namespace
+{
+bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch,
+                    size_t cus_of_device, bool any_rows)
 {
     const size_t rows = lc == 0 ? m : n;
     const size_t cols = lc == 0 ? n : m;
@@ -184,8 +191,10 @@ bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_pla
         a_kmajor     = b_kmajor;
         b_kmajor     = t;
     }
-    // K need not be whole K tiles: the persistent kernel cuts a partial last tile off
-    // itself, as long as the rows of a K-contiguous operand stay 16-byte aligned
+    // K need not be whole K tiles and no extent need be whole tiles: the persistent kernel cuts
+    // every ragged edge off itself.  What it needs is operands whose rows start on 16 bytes;
+    // one whose rows do not is copied first, which pays from copy_pays_flops per copied element on
+    // (the launch's own rule).
     const bool k_whole = k % 64 == 0;
     // Skinny against a large operand (decode-like: a few rows against 4096 x 4096 .. 28672
     // x 8192): the plans of the whole-K streaming kernel compete with the others by their
@@ -193,10 +202,24 @@ bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_pla
     launch_plan stream_best{};
     double      stream_us   = 0.0;
     const bool  have_stream = stream_plan(rows, cols, k, a_kmajor, b_kmajor, batch, cus_of_device, &stream_best, &stream_us);
-    if(k < 64 || rows % 8 != 0 || cols % 8 != 0 || rows < 16 || cols < 16
-       || (!k_whole && (a_kmajor || b_kmajor) && k % 8 != 0))
+    const bool   a_rows = (a_kmajor ? k : rows) % 8 == 0, b_rows = (b_kmajor ? k : cols) % 8 == 0;
+    const double copied = (a_rows ? 0.0 : static_cast<double>(rows * k)) + (b_rows ? 0.0 : static_cast<double>(cols * k));
+    const bool   pays   = copied == 0.0 || (k >= 128 && 2.0 * rows * cols * k >= (copy_pays_flops + 4.0) * copied);
+    const bool   regular = rows % 8 == 0 && cols % 8 == 0 && a_rows && b_rows;
+    // (a C that cannot take 16-byte pieces is not the persistent kernel's.  Where that or a copy
+    // comes in and 256 x 256 tiles cover half the chip, the nearest tuned entry's large tile serves
+    // as well or better: 3000 x 3000 x 3001, all row-major, 79 us against 89)
+    const bool   pieces  = cols % 8 == 0;
+    const size_t device  = cus_of_device != 0 ? cus_of_device : static_cast<size_t>(model_measured.compute_units);
+    const bool   few     = ceil_div(rows, size_t{256}) * ceil_div(cols, size_t{256}) * batch < device / 2;
+    const bool   takes   = regular || (any_rows && (few || (pieces && copied == 0.0))
+                              // (short sums into one or two million elements: the entry is a
+                              // streaming plan, which the estimate leaves to smaller problems:
+                              // 2001 x 1000 x 1000 21.0 us against 24.6)
+                              && !(copied == 0.0 && k <= 1024 && rows * cols > (size_t{1} << 20) && rows * cols <= (size_t{1} << 21)));
+    if(k < 64 || rows < 16 || cols < 16 || !pays || !takes)
     {
-        // shapes every direct kernel would only take through padded copies
+        // (the copies would cost more than the general kernel's own way of loading)
         if(have_stream)
         {
             *out = stream_best;
@@ -230,6 +253,10 @@ bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_pla
         {
             continue;
         }
+        if(v.pipeline == 5 && !pieces)
+        {
+            continue;
+        }
         const size_t bm = v.block_m, bn = v.block_n;
         if((bm % 128 != 0 && !a_kmajor) || (bn % 128 != 0 && !b_kmajor))
         {
@@ -248,14 +275,21 @@ bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_pla
         const size_t tm = ceil_div(rows, bm), tn = ceil_div(cols, bn), tiles = tm * tn * batch;
         const double tile_bytes = static_cast<double>(bm * bn) * 4.0;
         // only the persistent kernel takes ragged M, N or K as they are; the others run on
-        // padded copies of the operands that need them (two more launches)
-        double copies_us = 0.0;
-        if(v.pipeline != 5 && (rows % bm != 0 || cols % bn != 0 || !k_whole))
+        // padded copies of the operands that need them (one more launch)
+        double     copies_us = 0.0;
+        const bool edges     = v.pipeline == 5;
+        const bool copy_a    = !a_rows || (!edges && (rows % bm != 0 || !k_whole));
+        const bool copy_b    = !b_rows || (!edges && (cols % bn != 0 || !k_whole));
+        if(copy_a || copy_b)
         {
             const double k_pad = static_cast<double>(kt * 64);
-            const double elems = ((rows % bm != 0 || !k_whole ? static_cast<double>(tm * bm) * k_pad : 0.0)
-                                  + (cols % bn != 0 || !k_whole ? static_cast<double>(tn * bn) * k_pad : 0.0))
+            const double elems = ((copy_a ? static_cast<double>(tm * bm) * k_pad : 0.0)
+                                  + (copy_b ? static_cast<double>(tn * bn) * k_pad : 0.0))
                                  * static_cast<double>(batch);
+            if(!edges && 2.0 * rows * cols * k * batch < (copy_pays_flops + 4.0) * elems)
+            {
+                continue; // (the launch would take the general kernel instead)
+            }
             copies_us = launch_us + elems * 2.0 * 2.0 / model_measured.copy_bytes_per_us;
         }
         auto consider = [&](double t, int split) {
@@ -351,6 +385,23 @@ bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_pla
         found = true;
     }
     return found;
+}
+} // namespace
+
+bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch,
+                size_t cus_of_device)
+{
+    return estimated_plan(m, n, k, lc, la, lb, out, batch, cus_of_device, false);
+}
+
+// Any number of tokens against a weight (133 x 5560 x 10232), odd extents: the nearest tuned
+// entry knows neither how many tiles there are nor that a small operand is cheap to copy
+// (133 x 5560 x 10232
+// 134 -> 90 us, 250 x 1001 x 40001 814 -> 75, 2001 x 2001 x 16384 321 -> 185).  Same arithmetic, with the copies of the operands that need them priced in.
+bool model_plan_any_rows(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch,
+                         size_t cus_of_device)
+{
+    return estimated_plan(m, n, k, lc, la, lb, out, batch, cus_of_device, true);
 }
 
 bool stream_plan(size_t rows, size_t cols, size_t k, bool a_kmajor, bool b_kmajor, size_t batch, size_t cus_of_device,
@@ -512,7 +563,7 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     launch_plan plan;
     // the table was tuned on single GEMMs: a batch changes how many tiles there are to
     // spread, which is the model's business
-    if(batch > 1 && model_plan(m, n, k, lc, la, lb, &plan, batch, cus))
+    if(batch > 1 && model_plan_any_rows(m, n, k, lc, la, lb, &plan, batch, cus))
     {
         return plan;
     }
@@ -536,17 +587,25 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
             return plan;
         }
     }
-    // ... then the model for regular shapes, and the nearest tuned entry for the rest
-    if(model_plan(m, n, k, lc, la, lb, &plan, 1, cus))
+    // ... then the model, and the nearest tuned entry for the rest
+    if(model_plan_any_rows(m, n, k, lc, la, lb, &plan, 1, cus))
     {
         return plan;
     }
     // A skinny shape that neither has an entry nor suits the model (rows that are not 16-byte
     // aligned): the nearest tuned entry would be a large square's plan, 256 x 256 tiles
-    // for a handful of rows; the shape heuristic cuts K over the compute units instead.
-    if(std::min(m, n) <= 64 && std::max(m, n) >= 512)
+    // for a handful of rows.  The general kernel's 64 x 64 tile, K cut until there are three
+    // workgroups to a compute unit (8 x 3678 x 3817, odd K: 41.2 us on the 128 x 128 tile with
+    // 15 slices, 28.0 on this one with 12).
+    if(std::min(m, n) <= 128 && std::max(m, n) >= 512)
     {
-        return heuristic_plan(m, n, k, lc);
+        const size_t tiles = ceil_div(m, size_t{64}) * ceil_div(n, size_t{64}), steps = ceil_div(k, size_t{64});
+        const size_t units = cus != 0 ? cus : static_cast<size_t>(model_measured.compute_units);
+        plan.variant       = small_general_variant;
+        plan.swizzle       = 4;
+        plan.touch         = 0;
+        plan.split_k       = static_cast<int>(std::max<size_t>(1, std::min({3 * units / tiles, steps / 4, size_t{32}})));
+        return plan;
     }
     plan = select_plan_from(tuned_table, tuned_count, m, n, k, type_idx, lc, la, lb);
     // The nearest entry may be a small problem's, tuned onto the streaming kernel, which

@@ -123,11 +123,21 @@ bool find_exact(const tuned_entry* table, size_t count, size_t m, size_t n, size
 bool find_closest(const tuned_entry* table, size_t count, size_t m, size_t n, size_t k,
                   int type_group, int la, int lb, int lc, launch_plan* out);
 launch_plan heuristic_plan(size_t m, size_t n, size_t k, int lc);
+// Operations per element copied from which on padded copies of operands whose rows are not
+// aligned pay against the general kernel: about 100 rows against an odd weight (64 x 4096 x 4095:
+// 32.8 us copied, 20.5 by the general kernel; 96 rows 33.7 and 27.4; 133 x 5000 x 3001 43.1
+// and 278).
+constexpr double copy_pays_flops = 200.0;
+
 // Estimated-time choice among the compiled variants for a shape without a tuned entry;
 // false for shapes it does not cover (ragged K, odd extents).
 // cus: compute units of the GPU the plan is for (0: the GPU the constants were measured on).
 bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch = 1,
                 size_t cus = 0);
+// The same, also for extents whose rows do not start on 16 bytes (an odd number of tokens,
+// odd features): the operands that need it are copied first.
+bool model_plan_any_rows(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch = 1,
+                         size_t cus = 0);
 // The streaming kernel's plans alone (skinny shapes: one extent at most 128, or small ones:
 // at most 2^20 elements of C; K at least 256, a multiple of 8 where an operand is
 // K-contiguous), in kernel space (rows x cols, the operands' K-contiguity): the cheapest by

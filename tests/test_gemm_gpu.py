@@ -733,6 +733,51 @@ def test_partial_last_k_tile_on_the_persistent_kernel(loader):
                                              f"layouts C{lc} A{la} B{lb} {tname}: {e}") from None
 
 
+def test_rows_that_start_anywhere_on_the_persistent_kernel(loader):
+    """Operands whose rows do not start on 16 bytes, which the one-wave-per-SIMD kernel reads
+    from copies padded along the row only, and C that it cannot store (odd extents, odd batch
+    strides, a C that starts one element late), which goes to another kernel.  What lies before
+    and behind C stays as it was."""
+    import torch
+
+    solo = [v for v in loader.variants() if v.pipeline == 5]
+    cases = [  # M, N, K, batch, split field
+        (257, 511, 128, 1, 1),
+        (304, 769, 200, 1, 1),     # K-contiguous rows aligned: no copies in A row / B column
+        (255, 1001, 257, 1, 2),    # whole partial planes with odd rows, padded copies
+        (259, 513, 264, 3, 1),     # odd batch stride of C
+        (513, 523, 648, 1, -1),    # walk by K tile: parts in slots of their own
+        (4353, 257, 64, 1, -2),    # more tiles than workgroups, the last wave split
+        (256, 512, 128, 1, 1),     # whole tiles, C one element late
+        (257, 520, 193, 1, 1),     # A row / B column: both copied, C in place
+        (259, 512, 1000, 3, 2),    # batch entries of an odd stride
+        (513, 528, 649, 1, -1),
+    ]
+    for i, v in enumerate(solo):
+        for n, (M, N, K, batch, split) in enumerate(cases):
+            tname = list(TYPE_PAIRS)[(n + i) % 4]
+            din, dout = TYPE_PAIRS[tname]
+            for (lc, la, lb) in [l for l in [(0, 0, 1), (1, 1, 0), (0, 0, 0), (1, 1, 1)] if built_for(v, *l)]:
+                A = np.concatenate([O.init_matrix(M, K, la, din, seed=330 + b) for b in range(batch)])
+                B = np.concatenate([O.init_matrix(K, N, lb, din, seed=360 + b) for b in range(batch)])
+                size, before = M * N * batch, 9 if n % 2 == 0 and n < 7 else 8
+                buf = torch.full((size + 32,), float("nan"), dtype=torch_dtype(dout), device="cuda")
+                out = buf[before:before + size]
+                where = f"variant {v.index} {M}x{N}x{K} batch {batch} split {split} layouts C{lc} A{la} B{lb} {tname}"
+                rc = loader.run_variant(v.index, 4, split, out, to_device(A, din), to_device(B, din), M, N, K, lc, la,
+                                        lb, batch_count=batch)
+                assert rc == 0, where
+                torch.cuda.synchronize()
+                assert torch.isnan(buf[:before]).all() and torch.isnan(buf[before + size:]).all(), where
+                gpu = to_host(out.contiguous(), dout)
+                for b in range(batch):
+                    try:
+                        check_against_oracle(gpu[b * M * N:(b + 1) * M * N], A[b * M * K:(b + 1) * M * K],
+                                             B[b * K * N:(b + 1) * K * N], M, N, K, lc, la, lb, din, dout)
+                    except AssertionError as e:
+                        raise AssertionError(f"{where} entry {b}: {e}") from None
+
+
 def test_what_lies_past_k_does_not_reach_c(loader):
     """The columns of the last K tile past K must be zeros, not whatever follows in memory
     times zero: with infinities right behind a row's K columns (the next row's first
