@@ -215,8 +215,8 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     const bool   takes   = regular || (any_rows && (few || (pieces && copied == 0.0))
                               // (short sums into one or two million elements: the entry is a
                               // streaming plan, which the estimate leaves to smaller problems:
-                              // 2001 x 1000 x 1000 21.0 us against 24.6)
-                              && !(copied == 0.0 && k <= 1024 && rows * cols > (size_t{1} << 20) && rows * cols <= (size_t{1} << 21)));
+                              // 2001 x 1000 x 1000 21.0 us against 24.6, x 2000 30.8 against 42.0)
+                              && !(copied == 0.0 && k <= 4096 && rows * cols > (size_t{1} << 20) && rows * cols <= (size_t{1} << 21)));
     if(k < 64 || rows < 16 || cols < 16 || !pays || !takes)
     {
         // (the copies would cost more than the general kernel's own way of loading)
