@@ -760,7 +760,7 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
         return slices;
     };
     split_k = without_empty_slices(split_k);
-    const size_t split_tiles = tiles - tail_begin;
+    size_t split_tiles = tiles - tail_begin;
     if(tail_begin + split_tiles * static_cast<size_t>(split_k) > 0x7fffffffull)
     {
         split_k = 1;
@@ -779,7 +779,10 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
     }
     if(split_k == 1)
     {
-        tail_begin = 0;
+        // nothing is left to split (K of one step, or partial sums beyond the budget): the
+        // launch covers every tile, those of the last wave among them
+        tail_begin  = 0;
+        split_tiles = tiles;
     }
     if(split_k > 1)
     {

@@ -513,6 +513,19 @@ def test_split_tail_wave_agrees_with_oracle(loader):
                                          f"C{lc} A{la} B{lb}: {e}") from None
 
 
+@pytest.mark.parametrize("variant", [34, 18, 21])
+def test_split_tail_wave_of_a_single_k_step_covers_every_tile(loader, variant):
+    """A plan that asks for a split tail where K is one step long has nothing to split: all 289
+    tiles (more than the compute units of the GPU) are computed whole, those of the last wave
+    and those before it."""
+    v = loader.variants()[variant]
+    M, N, K = 17 * v.block_m, 17 * v.block_n, v.block_k
+    A, B = make_inputs(M, N, K, 0, 1, O.F16)
+    for split in (-2, -8):
+        gpu = run_gpu(loader, A, B, M, N, K, 0, 0, 1, O.F16, O.F16, variant=(v.index, 4, split))
+        check_against_oracle(gpu, A, B, M, N, K, 0, 0, 1, O.F16, O.F16)
+
+
 def test_mirrored_tile_walk_agrees_with_oracle(loader):
     """Negative swizzle: the tile walk runs in bands of tile columns instead of tile rows.
     Every pipeline, whole K, every tile split, split tail wave and (persistent kernel) the
