@@ -590,6 +590,22 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     // ... then the model, and the nearest tuned entry for the rest
     if(model_plan_any_rows(m, n, k, lc, la, lb, &plan, 1, cus))
     {
+        // The order of the K tiles within a tile is timed per weight, the estimate only knows
+        // groups of 8 from 300 MB on.  A number of rows that no table holds takes the order of
+        // the nearest entry where that has one and agrees on the tile and the split: 777 rows
+        // against 28672 x 8192 weights, groups of 4, B column-major 372 -> 356 us, row-major (where
+        // the estimate has no groups at all) 408 -> 366; 509 rows, in runs, 216 -> 213.  An entry
+        // without an order says less: 3001 x 20480 x 10240 is 1007 us in the estimate's groups
+        // of 8, 1126 without.
+        launch_plan nearest;
+        if((m % 8 != 0 || n % 8 != 0 || k % 8 != 0)
+           && (find_closest(tuned_table, tuned_count, m, n, k, group, la, lb, lc, &nearest)
+               || (group != 0 && find_closest(tuned_table, tuned_count, m, n, k, 0, la, lb, lc, &nearest)))
+           && nearest.variant == plan.variant && nearest.split_k == plan.split_k
+           && (plan_k_run(nearest.touch) > 0 || plan_k_group(nearest.touch) > 0))
+        {
+            plan.touch = nearest.touch;
+        }
         return plan;
     }
     // A skinny shape that neither has an entry nor suits the model (rows that are not 16-byte

@@ -229,6 +229,17 @@ static int check_select()
         if(tiles[r3.variant].pipeline == 7)
             return fail("select: 3 rows that are not K-contiguous must not stream");
     }
+    // a number of rows that no table holds takes the K order timed for the same weight (768 and
+    // 1024 rows: groups of 4 K tiles), in both layouts of B; a weight whose nearest entry has
+    // none keeps the estimate's groups of 8
+    {
+        const launch_plan q = select_plan(777, 28672, 8192, 2, 0, 0, 1), r = select_plan(777, 28672, 8192, 2, 0, 0, 0);
+        if(tiles[q.variant].pipeline != 5 || plan_k_group(q.touch) != 4 || plan_k_group(r.touch) != 4)
+            return fail("select: 777 rows take the K order of the nearest tuned row counts");
+        const launch_plan t = select_plan(3001, 20480, 10240, 2, 0, 0, 1);
+        if(tiles[t.variant].pipeline != 5 || plan_k_group(t.touch) != 8)
+            return fail("select: a weight without a timed K order keeps the estimate's");
+    }
     // next to 1024^3, whose entries run on the streaming kernel: K-contiguous rows that are
     // not 16-byte aligned must not inherit that plan
     {
