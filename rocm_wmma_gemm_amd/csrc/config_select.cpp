@@ -208,10 +208,12 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     const bool   regular = rows % 8 == 0 && cols % 8 == 0 && a_rows && b_rows;
     // (a C that cannot take 16-byte pieces is not the persistent kernel's.  Where that or a copy
     // comes in and 256 x 256 tiles cover half the chip, the nearest tuned entry's large tile serves
-    // as well or better: 3000 x 3000 x 3001, all row-major, 79 us against 89)
+    // as well or better: 3000 x 3000 x 3001, all row-major, 79 us against 89.  Counted for one entry
+    // of a batch: what the table would give 64 x 856 x 673 x 1014 is a small tile in 4 slices, 544 us,
+    // the estimate 243)
     const bool   pieces  = cols % 8 == 0;
     const size_t device  = cus_of_device != 0 ? cus_of_device : static_cast<size_t>(model_measured.compute_units);
-    const bool   few     = ceil_div(rows, size_t{256}) * ceil_div(cols, size_t{256}) * batch < device / 2;
+    const bool   few     = ceil_div(rows, size_t{256}) * ceil_div(cols, size_t{256}) < device / 2;
     const bool   takes   = regular || (any_rows && (few || (pieces && copied == 0.0))
                               // (short sums into one or two million elements: the entry is a
                               // streaming plan, which the estimate leaves to smaller problems:
@@ -587,8 +589,10 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
             return plan;
         }
     }
-    // ... then the model, and the nearest tuned entry for the rest
-    if(model_plan_any_rows(m, n, k, lc, la, lb, &plan, 1, cus))
+    // ... then the model, and the nearest tuned entry for the rest.  (Not for a batch: the model
+    // has declined it above, and one entry priced as if it had the chip to itself would have its K
+    // cut for nothing: 128 x 511 x 511 x 4001 in 8 slices, 2048 tiles before any cut.)
+    if(batch == 1 && model_plan_any_rows(m, n, k, lc, la, lb, &plan, 1, cus))
     {
         // The order of the K tiles within a tile is timed per weight, the estimate only knows
         // groups of 8 from 300 MB on.  A number of rows that no table holds takes the order of
@@ -613,9 +617,10 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     // for a handful of rows.  The general kernel's 64 x 64 tile, K cut until there are three
     // workgroups to a compute unit (8 x 3678 x 3817, odd K: 41.2 us on the 128 x 128 tile with
     // 15 slices, 28.0 on this one with 12).
+    // A batch brings workgroups of its own.
     if(std::min(m, n) <= 128 && std::max(m, n) >= 512)
     {
-        const size_t tiles = ceil_div(m, size_t{64}) * ceil_div(n, size_t{64}), steps = ceil_div(k, size_t{64});
+        const size_t tiles = ceil_div(m, size_t{64}) * ceil_div(n, size_t{64}) * batch, steps = ceil_div(k, size_t{64});
         const size_t units = cus != 0 ? cus : static_cast<size_t>(model_measured.compute_units);
         plan.variant       = small_general_variant;
         plan.swizzle       = 4;
@@ -624,6 +629,16 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
         return plan;
     }
     plan = select_plan_from(tuned_table, tuned_count, m, n, k, type_idx, lc, la, lb);
+    // (its cut along K was timed on one GEMM: a batch that fills the GPU with whole tiles has no use for it)
+    if(batch > 1 && plan.split_k > 1)
+    {
+        const model_variant& t     = model_variants[plan.variant];
+        const size_t         units = cus != 0 ? cus : static_cast<size_t>(model_measured.compute_units);
+        if(ceil_div(m, t.block_m) * ceil_div(n, t.block_n) * batch >= units)
+        {
+            plan.split_k = 1;
+        }
+    }
     // The nearest entry may be a small problem's, tuned onto the streaming kernel, which
     // wants 16-byte aligned rows of either kind: a
     // shape that does not fit takes the shape heuristic's plan instead.

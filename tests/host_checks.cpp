@@ -240,6 +240,20 @@ static int check_select()
         if(tiles[t.variant].pipeline != 5 || plan_k_group(t.touch) != 8)
             return fail("select: a weight without a timed K order keeps the estimate's");
     }
+    // a batch whose tiles fill the GPU by themselves is not cut along K, whether the model takes it,
+    // declines it or it is skinny
+    {
+        const struct { size_t m, n, k, batch; } full[] = {{511, 511, 4001, 128}, {1023, 1023, 4095, 32}, {1001, 701, 4097, 32},
+            {512, 512, 2001, 64}, {64, 4096, 4095, 64}, {531, 111, 572, 91}, {78, 810, 276, 73}, {512, 512, 512, 64}};
+        for(const auto& x : full)
+            for(int t = 0; t < 4; ++t)
+                for(int l = 0; l < 8; ++l)
+                    if(select_plan(x.m, x.n, x.k, t, l & 1, (l >> 1) & 1, l >> 2, x.batch, 256).split_k > 1)
+                        return fail("select: a batch that fills the GPU is cut along K");
+        // ... and one that does not still is
+        if(select_plan(46, 554, 2001, 0, 0, 0, 1, 3, 256).split_k < 2)
+            return fail("select: a small skinny batch is cut along K");
+    }
     // next to 1024^3, whose entries run on the streaming kernel: K-contiguous rows that are
     // not 16-byte aligned must not inherit that plan
     {
