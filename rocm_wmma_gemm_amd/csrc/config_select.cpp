@@ -614,18 +614,30 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     }
     // A skinny shape that neither has an entry nor suits the model (rows that are not 16-byte
     // aligned): the nearest tuned entry would be a large square's plan, 256 x 256 tiles
-    // for a handful of rows.  The general kernel's 64 x 64 tile, K cut until there are three
-    // workgroups to a compute unit (8 x 3678 x 3817, odd K: 41.2 us on the 128 x 128 tile with
-    // 15 slices, 28.0 on this one with 12).
+    // for a handful of rows.  The general kernel's small tiles, K cut until there are enough
+    // workgroups, all of them at once: three of 64 x 64 to a compute unit (8 x 3678 x 3817, odd K: 41.2 us
+    // on the 128 x 128 tile with 15 slices, 28.0 on this one with 12), two of 128 x 128.
+    // Up to 64 rows the 64 x 64 tile.  From 65 on it takes two rows of tiles, each of which reads all of
+    // the large operand, and the 128 x 128 tile is ahead where it covers the GPU: by its tiles
+    // alone (from one to two compute units on: 104 x 986 x 207 x 64 20.8 us, 39.2 on 64 x 64), or cut along a K
+    // of 2048 and more (80 x 8192 x 8191, B row-major 76 us against 124; 112 x 16000 x 3003 73 and 67;
+    // below that 80 x 8192 x 1001 29 and 25, and 80 x 1500 x 3003, where the slices end at 11, 24 and 19).
+    // Where both operands are K-contiguous, which the general kernel reads 16 bytes at a time
+    // whatever their alignment, reading the large one twice costs less: only from 64 MB of it on
+    // (97 x 13199 x 16899 311 us, 519 on 64 x 64; 85 x 1880 x 5811 32 and 27, 83 x 19047 x 566 32 and 20).
     // A batch brings workgroups of its own.
     if(std::min(m, n) <= 128 && std::max(m, n) >= 512)
     {
-        const size_t tiles = ceil_div(m, size_t{64}) * ceil_div(n, size_t{64}) * batch, steps = ceil_div(k, size_t{64});
         const size_t units = cus != 0 ? cus : static_cast<size_t>(model_measured.compute_units);
-        plan.variant       = small_general_variant;
+        const size_t small = ceil_div(m, size_t{64}) * ceil_div(n, size_t{64}) * batch;
+        const size_t large = ceil_div(m, size_t{128}) * ceil_div(n, size_t{128}) * batch;
+        const size_t cut   = std::max<size_t>(1, std::min({2 * units / large, k / 256, size_t{64}})); // 8 K steps of 32 a slice
+        const bool   once  = la == 0 && lb == 1 && batch == 1 && std::max(m, n) * k < (size_t{1} << 25);
+        const bool   wide  = std::min(m, n) > 64 && !once && (large * 2 >= units || (k >= 2048 && large * cut >= units));
+        plan.variant       = wide ? 0 : small_general_variant;
         plan.swizzle       = 4;
         plan.touch         = 0;
-        plan.split_k       = static_cast<int>(std::max<size_t>(1, std::min({3 * units / tiles, steps / 4, size_t{32}})));
+        plan.split_k       = static_cast<int>(wide ? cut : std::max<size_t>(1, std::min({3 * units / small, ceil_div(k, size_t{64}) / 4, size_t{32}})));
         return plan;
     }
     plan = select_plan_from(tuned_table, tuned_count, m, n, k, type_idx, lc, la, lb);

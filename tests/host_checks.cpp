@@ -240,6 +240,27 @@ static int check_select()
         if(tiles[t.variant].pipeline != 5 || plan_k_group(t.touch) != 8)
             return fail("select: a weight without a timed K order keeps the estimate's");
     }
+    // skinny shapes with unaligned rows: the general kernel's 64 x 64 tile for up to 64 rows and
+    // wherever 128 x 128 tiles would not cover the GPU, else those, all workgroups at once
+    {
+        const struct { size_t m, n, k, batch; int tile; } skinny[] = {{64, 8193, 8191, 1, 64}, {65, 8193, 8191, 1, 128}, {96, 4099, 13443, 1, 128},
+            {80, 1500, 1001, 1, 64}, {80, 1500, 3003, 1, 64}, {80, 1500, 8191, 1, 128}, {80, 8193, 1001, 1, 64}, {80, 28001, 1001, 1, 128}, {84, 25613, 23283, 1, 128},
+            {104, 987, 207, 64, 128}, {104, 987, 207, 2, 64}, {57, 829, 169, 64, 64}};
+        for(const auto& x : skinny)
+        {
+            // (A and B row-major, and the same problem transposed)
+            const launch_plan q = select_plan(x.m, x.n, x.k, 0, 0, 0, 0, x.batch, 256), r = select_plan(x.n, x.m, x.k, 0, 1, 1, 1, x.batch, 256);
+            const size_t      t = ((x.m + x.tile - 1) / x.tile) * ((x.n + x.tile - 1) / x.tile) * x.batch;
+            if(tiles[q.variant].pipeline != 0 || tiles[q.variant].bm != x.tile || tiles[q.variant].bn != x.tile
+               || q.split_k < 1 || (q.split_k > 1 && t * static_cast<size_t>(q.split_k) > (x.tile == 64 ? 768u : 512u)))
+                return fail("select: skinny shape with unaligned rows");
+            if(r.variant != q.variant || r.split_k != q.split_k)
+                return fail("select: skinny N like skinny M");
+        }
+        // both operands K-contiguous: 128 x 128 tiles from 64 MB of the large operand on
+        if(tiles[select_plan(80, 8192, 4095, 0, 0, 0, 1).variant].bm != 64 || tiles[select_plan(80, 8193, 4097, 0, 0, 0, 1).variant].bm != 128)
+            return fail("select: skinny shape with unaligned K-contiguous rows");
+    }
     // a batch whose tiles fill the GPU by themselves is not cut along K, whether the model takes it,
     // declines it or it is skinny
     {
