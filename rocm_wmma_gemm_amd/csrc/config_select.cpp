@@ -156,6 +156,13 @@ bool step_cost(const model_variant& v, double* step_us, double* item_us)
     return false;
 }
 
+// Padded copies where a row is not aligned, microseconds and bytes read and written per microsecond:
+// a launch that the GEMM waits for, and what pack_padded reaches on operands from HBM (2.8 GB in 0.67
+// ms; small ones that stay in the memory-side cache move at 5.6 TB/s).  At the 6 us and 3 TB/s
+// that regular extents are priced with, copies looked dear and the persistent kernel's large tiles cheap: 685 x 4488 x 1944
+// 49 us on 192 x 192, 37 on copies and 128 x 128; 1519 x 2232 x 4536 76 and 58.
+constexpr double copy_launch_us = 3.5, copy_bytes_per_us = 4.2e6;
+
 // the general kernel's smallest square tile, 64 x 64 x 64
 constexpr int small_general_variant = 34;
 
@@ -164,6 +171,23 @@ size_t ceil_div(size_t a, size_t b)
     return (a + b - 1) / b;
 }
 } // namespace
+
+operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b_kmajor, bool a_rows, bool b_rows,
+                             size_t block_m, size_t block_n, size_t block_k, bool edges)
+{
+    const size_t m_pad = ceil_div(m, edges ? 8 : block_m) * (edges ? 8 : block_m),
+                 n_pad = ceil_div(n, edges ? 8 : block_n) * (edges ? 8 : block_n), k_pad = ceil_div(k, block_k) * block_k;
+    operand_copies c;
+    c.a       = !a_rows || (!edges && !(k_pad == k && m_pad == m));
+    c.b       = !b_rows || (!edges && !(k_pad == k && n_pad == n));
+    c.lda     = a_kmajor ? (c.a ? k_pad : k) : (c.a ? m_pad : m);
+    c.ldb     = b_kmajor ? (c.b ? k_pad : k) : (c.b ? n_pad : n);
+    c.elems_a = !c.a ? 0 : c.lda * (!edges ? (a_kmajor ? m_pad : k_pad) : a_kmajor ? m : k);
+    c.elems_b = !c.b ? 0 : c.ldb * (!edges ? (b_kmajor ? n_pad : k_pad) : b_kmajor ? n : k);
+    const double copied = static_cast<double>(c.elems_a + c.elems_b);
+    c.pays              = copied > 0.0 && k >= 128 && 2.0 * m * n * k >= copy_pays_flops * copied;
+    return c;
+}
 
 // A plan from arithmetic instead of from the nearest tuned shape: for every compiled
 // variant of the two pipelines that serve regular shapes, and every way to split, the
@@ -193,9 +217,7 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     }
     // K need not be whole K tiles and no extent need be whole tiles: the persistent kernel cuts
     // every ragged edge off itself.  What it needs is operands whose rows start on 16 bytes;
-    // one whose rows do not is copied first, which pays from copy_pays_flops per copied element on
-    // (the launch's own rule).
-    const bool k_whole = k % 64 == 0;
+    // one whose rows do not is copied first, where that pays (padded_copies).
     // Skinny against a large operand (decode-like: a few rows against 4096 x 4096 .. 28672
     // x 8192): the plans of the whole-K streaming kernel compete with the others by their
     // estimates, and stand alone for the shapes the others would only take through copies.
@@ -203,8 +225,6 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     double      stream_us   = 0.0;
     const bool  have_stream = stream_plan(rows, cols, k, a_kmajor, b_kmajor, batch, cus_of_device, &stream_best, &stream_us);
     const bool   a_rows = (a_kmajor ? k : rows) % 8 == 0, b_rows = (b_kmajor ? k : cols) % 8 == 0;
-    const double copied = (a_rows ? 0.0 : static_cast<double>(rows * k)) + (b_rows ? 0.0 : static_cast<double>(cols * k));
-    const bool   pays   = copied == 0.0 || (k >= 128 && 2.0 * rows * cols * k >= (copy_pays_flops + 4.0) * copied);
     const bool   regular = rows % 8 == 0 && cols % 8 == 0 && a_rows && b_rows;
     // (a C that cannot take 16-byte pieces is not the persistent kernel's.  Where that or a copy
     // comes in and 256 x 256 tiles cover half the chip, the nearest tuned entry's large tile serves
@@ -214,14 +234,13 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     const bool   pieces  = cols % 8 == 0;
     const size_t device  = cus_of_device != 0 ? cus_of_device : static_cast<size_t>(model_measured.compute_units);
     const bool   few     = ceil_div(rows, size_t{256}) * ceil_div(cols, size_t{256}) < device / 2;
-    const bool   takes   = regular || (any_rows && (few || (pieces && copied == 0.0))
+    const bool   takes   = regular || (any_rows && (few || (pieces && a_rows && b_rows))
                               // (short sums into one or two million elements: the entry is a
                               // streaming plan, which the estimate leaves to smaller problems:
                               // 2001 x 1000 x 1000 21.0 us against 24.6, x 2000 30.8 against 42.0)
-                              && !(copied == 0.0 && k <= 4096 && rows * cols > (size_t{1} << 20) && rows * cols <= (size_t{1} << 21)));
-    if(k < 64 || rows < 16 || cols < 16 || !pays || !takes)
+                              && !(a_rows && b_rows && k <= 4096 && rows * cols > (size_t{1} << 20) && rows * cols <= (size_t{1} << 21)));
+    if(k < 64 || rows < 16 || cols < 16 || !takes)
     {
-        // (the copies would cost more than the general kernel's own way of loading)
         if(have_stream)
         {
             *out = stream_best;
@@ -246,6 +265,7 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     const size_t     kt            = ceil_div(k, size_t{64});
     double           best          = 0.0;
     bool             found         = false;
+    bool             best_copies_large = false; // the cheapest tiled plan runs on a copy of the larger operand
     const int        count         = static_cast<int>(sizeof(model_variants) / sizeof(model_variants[0]));
     for(int i = 0; i < count; ++i)
     {
@@ -278,21 +298,20 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
         const double tile_bytes = static_cast<double>(bm * bn) * 4.0;
         // only the persistent kernel takes ragged M, N or K as they are; the others run on
         // padded copies of the operands that need them (one more launch)
-        double     copies_us = 0.0;
-        const bool edges     = v.pipeline == 5;
-        const bool copy_a    = !a_rows || (!edges && (rows % bm != 0 || !k_whole));
-        const bool copy_b    = !b_rows || (!edges && (cols % bn != 0 || !k_whole));
-        if(copy_a || copy_b)
+        double               copies_us = 0.0;
+        const operand_copies copies    = padded_copies(rows, cols, k, a_kmajor, b_kmajor, a_rows, b_rows, bm, bn, 64, v.pipeline == 5);
+        if(copies.a || copies.b)
         {
-            const double k_pad = static_cast<double>(kt * 64);
-            const double elems = ((copy_a ? static_cast<double>(tm * bm) * k_pad : 0.0)
-                                  + (copy_b ? static_cast<double>(tn * bn) * k_pad : 0.0))
-                                 * static_cast<double>(batch);
-            if(!edges && 2.0 * rows * cols * k * batch < (copy_pays_flops + 4.0) * elems)
+            const double elems = static_cast<double>(copies.elems_a + copies.elems_b);
+            if(regular ? 2.0 * rows * cols * k < copy_pays_flops * elems : !copies.pays)
             {
-                continue; // (the launch would take the general kernel instead)
+                continue; // (the launch takes the general kernel instead)
             }
-            copies_us = launch_us + elems * 2.0 * 2.0 / model_measured.copy_bytes_per_us;
+            // (regular extents are priced as in the fit of the constants.  Below a K of 128 nothing is
+            // copied for them and the launch takes the general kernel's tile of the same size: 128 x 576 x 64
+            // 8.1 us, 8.5 by the nearest entry)
+            const double bytes = elems * static_cast<double>(batch) * 4.0;
+            copies_us          = regular ? launch_us + bytes / model_measured.copy_bytes_per_us : copy_launch_us + bytes / copy_bytes_per_us;
         }
         auto consider = [&](double t, int split) {
             t += copies_us;
@@ -300,6 +319,7 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
             {
                 found        = true;
                 best         = t;
+                best_copies_large = cols >= rows ? copies.b : copies.a;
                 out->variant = i;
                 out->swizzle = 4;
                 out->split_k = split;
@@ -365,7 +385,8 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     // the streaming plan's workgroups all run at once: the estimates are closer to each
     // other than to the truth where they need a second pass over the compute units
     // (128 x 14336 x 4096: 34.5 us streamed, 29.2 tiled; 128 x 8192 x 8192, one pass, 30.3
-    // against 37.4).
+    // against 37.4), or where the tiled plan would copy the large operand (101 x 22336 x 7808,
+    // B row-major: 118 us streamed, 220 on a copy).
     bool one_pass = false;
     if(have_stream)
     {
@@ -377,7 +398,8 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     }
     const size_t skinny  = std::min(rows, cols);
     const bool   compete = skinny <= 64 || (skinny <= 128 && one_pass)
-                         || (rows * cols <= (size_t{1} << 20) && k <= 4096);
+                         || (rows * cols <= (size_t{1} << 20) && k <= 4096)
+                         || (!regular && skinny <= 128 && best_copies_large);
     // (no tiled plan moves A and B faster than operand_bytes_per_us, which is what bounds the
     // skinny shapes; the estimates above rank the tiled plans among themselves without it)
     const double tiled_us = std::max(best, launch_us + operand_us);

@@ -129,6 +129,22 @@ launch_plan heuristic_plan(size_t m, size_t n, size_t k, int lc);
 // and 278).
 constexpr double copy_pays_flops = 200.0;
 
+// The padded copies that a direct-to-LDS tile needs of the operands of one problem, in kernel
+// space: what the launch makes of them and what the estimate prices.
+struct operand_copies
+{
+    bool   a, b; // which operands are copied ...
+    size_t lda, ldb; // ... their leading dimensions, copied or not ...
+    size_t elems_a, elems_b; // ... and the elements of a copy, per batch entry (0: none)
+    bool   pays; // there is something to copy and the GEMM is large next to it
+};
+// a_rows, b_rows: the operand's rows start on 16 bytes.  edges: the tile's kernel cuts ragged edges off
+// itself (the persistent one), so that only an operand whose rows are not aligned is copied, its
+// rows padded (a K-contiguous one's to whole K tiles) and their number left as it is; every other
+// kernel needs whole tiles.
+operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b_kmajor, bool a_rows, bool b_rows,
+                             size_t block_m, size_t block_n, size_t block_k, bool edges);
+
 // Estimated-time choice among the compiled variants for a shape without a tuned entry;
 // false for shapes it does not cover (ragged K, odd extents).
 // cus: compute units of the GPU the plan is for (0: the GPU the constants were measured on).

@@ -668,37 +668,26 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
             // an operand that needs it is copied: one whose rows are aligned and whose
             // extents are whole tiles stays where it is (a skinny GEMM pads its small
             // operand and streams the big one from where it lies).
-            // The persistent kernel cuts ragged edges off itself: only an operand whose rows
-            // are not aligned is copied, its rows padded to 16 bytes (a K-contiguous one's to
-            // whole K tiles) and their number left as it is.
-            const bool   edges = dv.pipeline == 5;
-            const size_t m_pad = round_up(p.M, edges ? 8 : dv.block_m), n_pad = round_up(p.N, edges ? 8 : dv.block_n),
-                         k_pad = round_up(p.K, dv.block_k);
+            const bool   edges  = dv.pipeline == 5;
             const bool   a_rows = aligned16(p.A) && (p.a_kmajor ? p.K : p.M) % 8 == 0
                                 && (p.batch == 1 || p.stride_a % 8 == 0);
             const bool   b_rows = aligned16(p.B) && (p.b_kmajor ? p.K : p.N) % 8 == 0
                                 && (p.batch == 1 || p.stride_b % 8 == 0);
-            copy_a = !a_rows || (!edges && !(k_pad == p.K && m_pad == p.M));
-            copy_b = !b_rows || (!edges && !(k_pad == p.K && n_pad == p.N));
-            const size_t plda = !copy_a ? lda : p.a_kmajor ? k_pad : m_pad;
-            const size_t pldb = !copy_b ? ldb : p.b_kmajor ? k_pad : n_pad;
-            const size_t pa = plda * (!edges ? (p.a_kmajor ? m_pad : k_pad) : p.a_kmajor ? p.M : p.K);
-            const size_t pb = pldb * (!edges ? (p.b_kmajor ? n_pad : k_pad) : p.b_kmajor ? p.N : p.K);
-            const size_t copied = (copy_a ? pa : 0) + (copy_b ? pb : 0);
-            pack_bytes = round_up(copied * p.batch * in_bytes, 256);
-            // padding pays when the GEMM is large next to the copy
-            const bool pays = copied > 0 && p.K >= 128
-                              && 2.0 * p.M * p.N * p.K / static_cast<double>(copied) >= copy_pays_flops;
-            if(pays && spans_fit(dv, p.a_kmajor, p.b_kmajor, plda, pldb, edges ? 31 : 32)
+            const operand_copies copies = padded_copies(p.M, p.N, p.K, p.a_kmajor, p.b_kmajor, a_rows, b_rows,
+                                                        dv.block_m, dv.block_n, dv.block_k, edges);
+            copy_a     = copies.a;
+            copy_b     = copies.b;
+            pack_bytes = round_up((copies.elems_a + copies.elems_b) * p.batch * in_bytes, 256);
+            if(copies.pays && spans_fit(dv, p.a_kmajor, p.b_kmajor, copies.lda, copies.ldb, edges ? 31 : 32)
                && pack_bytes <= workspace_limit_bytes / 2)
             {
                 packed   = true;
                 k_tail   = edges ? static_cast<int>(p.K % dv.block_k) : 0;
-                lda      = plda;
-                ldb      = pldb;
-                k_kernel = k_pad;
-                stride_a = copy_a ? pa : p.stride_a;
-                stride_b = copy_b ? pb : p.stride_b;
+                lda      = copies.lda;
+                ldb      = copies.ldb;
+                k_kernel = round_up(p.K, dv.block_k);
+                stride_a = copy_a ? copies.elems_a : p.stride_a;
+                stride_b = copy_b ? copies.elems_b : p.stride_b;
                 mode     = static_cast<int>(device::load_mode::vec_guarded); // guarded C stores
             }
             else

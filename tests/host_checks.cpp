@@ -134,6 +134,12 @@ static int check_select()
 #include "variants.def"
     };
 #undef RWG_VARIANT
+    struct block { int bm, bn, bk, pipeline; };
+#define RWG_VARIANT(IDX, BM, BN, BK, WM, WN, PIPE) {BM, BN, BK, PIPE},
+    const block blocks[] = {
+#include "variants.def"
+    };
+#undef RWG_VARIANT
     launch_plan p;
     // 3584^3: 196 tiles of 256 x 256 in one wave, not 361 of 192 x 192 in two
     if(!model_plan(3584, 3584, 3584, 0, 0, 1, &p) || tiles[p.variant].bm != 256 || tiles[p.variant].bn != 256
@@ -274,6 +280,34 @@ static int check_select()
         // ... and one that does not still is
         if(select_plan(46, 554, 2001, 0, 0, 0, 1, 3, 256).split_k < 2)
             return fail("select: a small skinny batch is cut along K");
+    }
+    // the estimate and the launch agree on the padded copies: no plan asks for a direct-to-LDS tile
+    // whose copies do not pay, which the launch would replace by the general kernel
+    {
+        const struct { size_t m, n, k; } ragged[] = {{256, 256, 193}, {257, 255, 193}, {300, 700, 129}, {200, 200, 4001}, {129, 4097, 1001},
+            {193, 193, 257}, {129, 300, 1000}, {208, 208, 2056}, {131, 131, 8191}, {1000, 1001, 1003}, {145, 777, 333}};
+        for(const auto& x : ragged)
+            for(int l = 0; l < 8; ++l)
+            {
+                const int         lc = l & 1, la = (l >> 1) & 1, lb = l >> 2;
+                const launch_plan q  = select_plan(x.m, x.n, x.k, 0, lc, la, lb);
+                const auto&       t  = blocks[q.variant];
+                if(t.pipeline == 0 || t.pipeline == 7)
+                    continue;
+                const size_t rows = lc == 0 ? x.m : x.n, cols = lc == 0 ? x.n : x.m;
+                const bool   ak = lc == 0 ? la == 0 : lb == 1, bk = lc == 0 ? lb == 1 : la == 0;
+                const auto   c = padded_copies(rows, cols, x.k, ak, bk, (ak ? x.k : rows) % 8 == 0, (bk ? x.k : cols) % 8 == 0,
+                                               t.bm, t.bn, t.bk, t.pipeline == 5);
+                if((c.a || c.b) && !c.pays && model_plan_any_rows(x.m, x.n, x.k, lc, la, lb, &p))
+                    return fail("select: a tile whose padded copies do not pay");
+            }
+        // what is copied: rows padded to 16 bytes or whole K tiles for the persistent kernel, whole tiles for the others
+        const auto e = padded_copies(257, 520, 193, true, false, false, true, 256, 256, 64, true);
+        if(!e.a || e.b || e.lda != 256 || e.ldb != 520 || e.elems_a != 257 * 256 || e.elems_b != 0 || !e.pays)
+            return fail("copies: the persistent kernel");
+        const auto w = padded_copies(257, 520, 193, true, false, false, true, 128, 128, 64, false);
+        if(!w.a || !w.b || w.lda != 256 || w.ldb != 640 || w.elems_a != 384 * 256 || w.elems_b != 640 * 256 || w.pays)
+            return fail("copies: whole tiles");
     }
     // next to 1024^3, whose entries run on the streaming kernel: K-contiguous rows that are
     // not 16-byte aligned must not inherit that plan
