@@ -156,12 +156,15 @@ bool step_cost(const model_variant& v, double* step_us, double* item_us)
     return false;
 }
 
-// Padded copies where a row is not aligned, microseconds and bytes read and written per microsecond:
-// a launch that the GEMM waits for, and what pack_padded reaches on operands from HBM (2.8 GB in 0.67
-// ms; small ones that stay in the memory-side cache move at 5.6 TB/s).  At the 6 us and 3 TB/s
-// that regular extents are priced with, copies looked dear and the persistent kernel's large tiles cheap: 685 x 4488 x 1944
-// 49 us on 192 x 192, 37 on copies and 128 x 128; 1519 x 2232 x 4536 76 and 58.
-constexpr double copy_launch_us = 3.5, copy_bytes_per_us = 4.2e6;
+// Padded copies where a row is not aligned, in microseconds: a launch that the GEMM waits for, and the
+// bytes read and written, 5.6 TB/s while they are few, 4.2 over 2.8 GB.  At the 6 us and 3 TB/s
+// that regular extents are priced with, copies looked dear and the persistent kernel's large tiles
+// cheap: 685 x 4488 x 1944 49 us on 192 x 192, 37 on copies and 128 x 128; 1519 x 2232 x 4536 76 and 58.
+double unaligned_copies_us(double bytes)
+{
+    const double knee = 48.0 * 1024 * 1024;
+    return 3.5 + std::min(bytes, knee) / 5.6e6 + std::max(bytes - knee, 0.0) / 3.8e6;
+}
 
 // the general kernel's smallest square tile, 64 x 64 x 64
 constexpr int small_general_variant = 34;
@@ -234,11 +237,10 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     const bool   pieces  = cols % 8 == 0;
     const size_t device  = cus_of_device != 0 ? cus_of_device : static_cast<size_t>(model_measured.compute_units);
     const bool   few     = ceil_div(rows, size_t{256}) * ceil_div(cols, size_t{256}) < device / 2;
-    const bool   takes   = regular || (any_rows && (few || (pieces && a_rows && b_rows))
-                              // (short sums into one or two million elements: the entry is a
-                              // streaming plan, which the estimate leaves to smaller problems:
-                              // 2001 x 1000 x 1000 21.0 us against 24.6, x 2000 30.8 against 42.0)
-                              && !(a_rows && b_rows && k <= 4096 && rows * cols > (size_t{1} << 20) && rows * cols <= (size_t{1} << 21)));
+    // (and copies, one more launch, need a K of 256: 441 x 806 x 150 13.4 us with them, 9.9 by the general
+    // kernel; 1018 x 222 x 201 13.7 and 12.7; 254 x 773 x 285 14.1 and 15.3; 608 x 177 x 382 14.2 and 17.5)
+    const bool   rows_ok = a_rows && b_rows;
+    const bool   takes   = regular || (any_rows && (rows_ok ? few || pieces : few && k >= 256));
     if(k < 64 || rows < 16 || cols < 16 || !takes)
     {
         if(have_stream)
@@ -311,7 +313,7 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
             // copied for them and the launch takes the general kernel's tile of the same size: 128 x 576 x 64
             // 8.1 us, 8.5 by the nearest entry)
             const double bytes = elems * static_cast<double>(batch) * 4.0;
-            copies_us          = regular ? launch_us + bytes / model_measured.copy_bytes_per_us : copy_launch_us + bytes / copy_bytes_per_us;
+            copies_us          = regular ? launch_us + bytes / model_measured.copy_bytes_per_us : unaligned_copies_us(bytes);
         }
         auto consider = [&](double t, int split) {
             t += copies_us;
@@ -403,7 +405,15 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     // (no tiled plan moves A and B faster than operand_bytes_per_us, which is what bounds the
     // skinny shapes; the estimates above rank the tiled plans among themselves without it)
     const double tiled_us = std::max(best, launch_us + operand_us);
-    if(have_stream && (!found || (stream_us < tiled_us && compete)))
+    // (ragged extents with a longer K, where tiles are part empty and some plans copy: from HBM the streaming
+    // plan takes 1.6 times its estimate, the tiled ones less than theirs, and the two are level
+    // where the estimates are 1 to 2.  391 timed pairs with one workgroup to a streaming tile: 0.86 of
+    // the tiled time beyond that ratio, 171 x 1088 x 4800 14 us and 25, 141 x 5440 x 7744 44 and 69; 1.22 below
+    // it.  Not for its 16-wide tiles, 1.15, nor past a K of 8192: 189 x 2048 x 14120 65 us, 54 tiled)
+    const bool stream_late = !regular && skinny > 128 && k > 4096 && k <= 8192 && have_stream && stream_best.split_k == 1
+                             && model_variants[stream_best.variant].block_m > 16 && model_variants[stream_best.variant].block_n > 16
+                             && 2.0 * stream_us < tiled_us;
+    if(have_stream && (!found || stream_late || (stream_us < tiled_us && compete)))
     {
         *out  = stream_best;
         found = true;
@@ -616,21 +626,37 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     // cut for nothing: 128 x 511 x 511 x 4001 in 8 slices, 2048 tiles before any cut.)
     if(batch == 1 && model_plan_any_rows(m, n, k, lc, la, lb, &plan, 1, cus))
     {
-        // The order of the K tiles within a tile is timed per weight, the estimate only knows
-        // groups of 8 from 300 MB on.  A number of rows that no table holds takes the order of
-        // the nearest entry where that has one and agrees on the tile and the split: 777 rows
-        // against 28672 x 8192 weights, groups of 4, B column-major 372 -> 356 us, row-major (where
-        // the estimate has no groups at all) 408 -> 366; 509 rows, in runs, 216 -> 213.  An entry
-        // without an order says less: 3001 x 20480 x 10240 is 1007 us in the estimate's groups
-        // of 8, 1126 without.
         launch_plan nearest;
         if((m % 8 != 0 || n % 8 != 0 || k % 8 != 0)
            && (find_closest(tuned_table, tuned_count, m, n, k, group, la, lb, lc, &nearest)
-               || (group != 0 && find_closest(tuned_table, tuned_count, m, n, k, 0, la, lb, lc, &nearest)))
-           && nearest.variant == plan.variant && nearest.split_k == plan.split_k
-           && (plan_k_run(nearest.touch) > 0 || plan_k_group(nearest.touch) > 0))
+               || (group != 0 && find_closest(tuned_table, tuned_count, m, n, k, 0, la, lb, lc, &nearest))))
         {
-            plan.touch = nearest.touch;
+            // A short sum into a million or two elements of C is where the estimate knows least: it prices
+            // neither the general kernel nor, beyond a million, the streaming one, which both take
+            // ragged extents without copies.  An entry of theirs goes before a tiled plan (1134 x 1032 x 1272,
+            // streaming, 18 us and 25 by the estimate, 774 x 2104 x 1104 22 and 26; 1544 x 900 x 608, general, 12
+            // and 18, 290 x 4416 x 1792 29 and 37).  Not further: 269 x 4808 x 3816 50 us and 39,
+            // 2657 x 1344 x 1088 39 and 24.
+            const size_t elements = m * n;
+            if((model_variants[nearest.variant].pipeline == 7 || model_variants[nearest.variant].pipeline == 0)
+               && model_variants[plan.variant].pipeline != 7 && nearest.split_k <= 1 && std::min(m, n) > 128
+               && elements > (size_t{1} << 20) && elements <= (size_t{1} << 21) && k <= 2048
+               && streaming_takes(m, n, k, lc, la, lb))
+            {
+                return nearest;
+            }
+            // The order of the K tiles within a tile is timed per weight, the estimate only knows
+            // groups of 8 from 300 MB on.  A number of rows that no table holds takes the order of
+            // the nearest entry where that has one and agrees on the tile and the split: 777 rows
+            // against 28672 x 8192 weights, groups of 4, B column-major 372 -> 356 us, row-major (where
+            // the estimate has no groups at all) 408 -> 366; 509 rows, in runs, 216 -> 213.  An entry
+            // without an order says less: 3001 x 20480 x 10240 is 1007 us in the estimate's groups
+            // of 8, 1126 without.
+            if(nearest.variant == plan.variant && nearest.split_k == plan.split_k
+               && (plan_k_run(nearest.touch) > 0 || plan_k_group(nearest.touch) > 0))
+            {
+                plan.touch = nearest.touch;
+            }
         }
         return plan;
     }

@@ -309,6 +309,28 @@ static int check_select()
         if(!w.a || !w.b || w.lda != 256 || w.ldb != 640 || w.elems_a != 384 * 256 || w.elems_b != 640 * 256 || w.pays)
             return fail("copies: whole tiles");
     }
+    // a number of rows that is no multiple of 8, rows of the operands aligned: the streaming and the general
+    // kernel's tuned entries for short sums into one to two million elements, the streaming plan for
+    // up to one million and a K of 8192, the tiled estimate beyond
+    {
+        const struct { size_t m, n, k; int type, lb, pipeline; } near[] = {{774, 2104, 1104, 0, 1, 7}, {290, 4416, 1792, 3, 1, 0}, {171, 1088, 4800, 1, 1, 7},
+            {141, 5440, 7744, 3, 0, 7}, {289, 1728, 10816, 0, 0, 5}, {269, 4808, 3816, 1, 1, 5}, {143, 3328, 5760, 3, 1, 6}};
+        for(const auto& x : near)
+            if(tiles[select_plan(x.m, x.n, x.k, x.type, 0, 0, x.lb).variant].pipeline != x.pipeline)
+                return fail("select: an odd number of rows, aligned operands");
+        // (with K past 2048 there is no step at two million elements of C)
+        for(size_t k : {2056, 3000, 4000})
+        {
+            const launch_plan u = select_plan(2001, 1040, k, 0, 0, 0, 1), w = select_plan(2001, 1056, k, 0, 0, 0, 1);
+            if(u.variant != w.variant || u.split_k != w.split_k)
+                return fail("select: a step in the plan at two million elements of C");
+        }
+        // a short K does not pay for copies of unaligned rows
+        for(int l = 0; l < 8; ++l)
+            if(tiles[select_plan(441, 806, 150, 2, l & 1, (l >> 1) & 1, l >> 2).variant].pipeline == 5
+               || tiles[select_plan(441, 807, 151, 2, l & 1, (l >> 1) & 1, l >> 2).variant].pipeline != 0)
+                return fail("select: copies for a short K");
+    }
     // next to 1024^3, whose entries run on the streaming kernel: K-contiguous rows that are
     // not 16-byte aligned must not inherit that plan
     {
