@@ -175,6 +175,14 @@ size_t ceil_div(size_t a, size_t b)
 }
 } // namespace
 
+bool keeps_small_tile(size_t m, size_t n, size_t batch, int block_m, int block_n, size_t cus)
+{
+    const size_t units  = cus != 0 ? cus : static_cast<size_t>(model_measured.compute_units);
+    const bool   skinny = std::min(m, n) <= 128 && std::max(m, n) >= 512;
+    return block_m * block_n <= 64 * 64
+           && (skinny || std::min(m, n) <= 64 || ceil_div(m, size_t{128}) * ceil_div(n, size_t{128}) * batch < units);
+}
+
 operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b_kmajor, bool a_rows, bool b_rows,
                              size_t block_m, size_t block_n, size_t block_k, bool edges)
 {

@@ -145,6 +145,13 @@ struct operand_copies
 operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b_kmajor, bool a_rows, bool b_rows,
                              size_t block_m, size_t block_n, size_t block_k, bool edges);
 
+// Whether a plan of the general kernel keeps its tile where it reads the operands a few bytes at
+// a time, or goes to the 128 x 128 tile: a larger tile does not fit its registers then, the 64 x 64 tile
+// is the faster one until there are 128 x 128 tiles for every compute unit (645 x 584 x 173 x 3, 90 of them, 8.3
+// us and 11.2; 1048 x 373 x 723 x 16, 432 of them, 129 and 42; up to 64 rows it reads nothing twice
+// and stays).  Skinny problems have been weighed by select_plan.
+bool keeps_small_tile(size_t m, size_t n, size_t batch, int block_m, int block_n, size_t cus);
+
 // Estimated-time choice among the compiled variants for a shape without a tuned entry;
 // false for shapes it does not cover (ragged K, odd extents).
 // cus: compute units of the GPU the plan is for (0: the GPU the constants were measured on).

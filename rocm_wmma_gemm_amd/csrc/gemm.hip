@@ -1067,10 +1067,9 @@ int run(int type_idx, const launch_plan* forced, void* C, void* A, void* B, size
         // Same rule as in launch() for a staged variant picked directly: misaligned
         // operands go through the small tile.  A direct variant is left alone here:
         // launch() decides between padded copies and the staged kernels.
-        // (so is the 64 x 64 tile small enough, which only skinny shapes are sent to)
         const variant_desc& v    = variant_at(plan.variant);
         const int           mode = pick_mode(p, v, plan.split_k);
-        if(mode == static_cast<int>(device::load_mode::scalar) && v.block_m * v.block_n > 64 * 64)
+        if(mode == static_cast<int>(device::load_mode::scalar) && !keeps_small_tile(p.M, p.N, p.batch, v.block_m, v.block_n, compute_units_of_current_device()))
         {
             plan.variant = 0;
         }

@@ -281,6 +281,11 @@ static int check_select()
         if(select_plan(46, 554, 2001, 0, 0, 0, 1, 3, 256).split_k < 2)
             return fail("select: a small skinny batch is cut along K");
     }
+    // unaligned rows on the general kernel: 64 x 64 tiles until 128 x 128 ones cover the GPU, nothing larger
+    if(!keeps_small_tile(645, 584, 3, 64, 64, 256) || keeps_small_tile(1048, 373, 16, 64, 64, 256) || !keeps_small_tile(1048, 373, 16, 64, 64, 512)
+       || keeps_small_tile(645, 584, 3, 128, 64, 256) || !keeps_small_tile(64, 500, 128, 64, 64, 256) || !keeps_small_tile(100, 33000, 1, 64, 64, 256)
+       || keeps_small_tile(65, 500, 64, 64, 64, 256))
+        return fail("general kernel: tile for unaligned rows");
     // the estimate and the launch agree on the padded copies: no plan asks for a direct-to-LDS tile
     // whose copies do not pay, which the launch would replace by the general kernel
     {

@@ -791,6 +791,41 @@ def test_rows_that_start_anywhere_on_the_persistent_kernel(loader):
                         raise AssertionError(f"{where} entry {b}: {e}") from None
 
 
+@pytest.mark.parametrize("M,N,K,batch,type_name,layouts,route", [
+    # route: pipeline, tile rows and whether K is cut, as the dispatcher picks them
+    (133, 552, 1032, 1, "f16_f16", (0, 0, 0), (7, 16, False)),      # streaming estimate, ragged rows
+    (250, 1001, 4001, 1, "f32_bf16", (0, 0, 1), (6, 128, True)),    # odd C, copies of both, K cut
+    (333, 776, 2049, 1, "bf16_bf16", (0, 1, 0), (6, 128, True)),    # A column-major with an odd M, copied
+    (511, 511, 513, 4, "f16_f16", (0, 0, 1), (6, 128, False)),      # a batch, odd strides, copies
+    (856, 673, 1014, 16, "f32_bf16", (0, 1, 0), (6, 128, False)),   # a batch that fills the GPU: not cut
+    (1289, 520, 8200, 1, "f16_f16", (0, 0, 1), (5, 192, True)),     # persistent kernel, ragged M and N
+    (80, 1500, 1001, 1, "f32_f16", (0, 0, 0), (0, 64, True)),       # skinny, general kernel's small tile
+    (100, 4099, 4099, 1, "f16_f16", (0, 0, 0), (0, 128, True)),     # skinny, its large tile
+    (4099, 100, 4099, 1, "f16_f16", (1, 1, 1), (0, 128, True)),     # the same transposed
+    (104, 986, 207, 24, "f32_f16", (1, 1, 0), (0, 128, False)),     # a skinny batch
+    (441, 806, 150, 1, "bf16_bf16", (1, 0, 1), (0, 64, False)),     # too short a K for copies
+    (171, 1088, 4800, 1, "f32_f16", (0, 0, 1), (7, 32, False)),     # streaming estimate, K past 4096
+    (774, 2104, 1104, 1, "f16_f16", (0, 0, 1), (7, 64, False)),     # streaming entry, two million elements
+    (1544, 900, 608, 1, "bf16_bf16", (0, 0, 1), (0, 128, False)),   # general kernel's entry, 16-byte loads
+    (1048, 373, 723, 16, "f16_f16", (0, 1, 0), (None, None, None)),  # (through the tile rule of unaligned rows)
+])
+def test_unaligned_extents_through_the_default_dispatch(loader, M, N, K, batch, type_name, layouts, route):
+    """Extents that are no multiples of 8, on each route the dispatcher has for them: the plan is the
+    intended one and C is right in every batch entry."""
+    lc, la, lb = layouts
+    din, dout = TYPE_PAIRS[type_name]
+    variant, _, split = loader.select(M, N, K, list(TYPE_PAIRS).index(type_name), lc, la, lb, batch)
+    if route[0] is not None:
+        v = loader.variants()[variant]
+        assert (v.pipeline, v.block_m, split not in (0, 1)) == route, (v, split)
+    A = np.concatenate([O.init_matrix(M, K, la, din, seed=410 + b) for b in range(batch)])
+    B = np.concatenate([O.init_matrix(K, N, lb, din, seed=450 + b) for b in range(batch)])
+    gpu = run_gpu(loader, A, B, M, N, K, lc, la, lb, din, dout, batch=batch)
+    for b in range(batch):
+        check_against_oracle(gpu[b * M * N:(b + 1) * M * N], A[b * M * K:(b + 1) * M * K],
+                             B[b * K * N:(b + 1) * K * N], M, N, K, lc, la, lb, din, dout)
+
+
 def test_what_lies_past_k_does_not_reach_c(loader):
     """The columns of the last K tile past K must be zeros, not whatever follows in memory
     times zero: with infinities right behind a row's K columns (the next row's first
