@@ -190,6 +190,9 @@ int rocm_wmma_gemm_workspace_release(void);
  *     ROCM_WMMA_GEMM_ERR_SCRATCH and enqueues nothing (of the shapes the library is
  *     tuned for: K = 65536 at M = N = 1024, which wants 128 MiB of partial tiles, and
  *     (4095, 5121, 3001), which wants 56 MiB of padded copies plus its partial tiles).
+ *     Extents whose rows do not start on 16 bytes have a second plan, the nearest tuned
+ *     shape's, which needs less or none: it is tried before the call fails, so that such a
+ *     call may run on another plan here than through the other entry points, and slower.
  *     Calls that need no scratch memory (whole tiles, no split) have no size limit.
  *   - The first call on a GPU looks the array's address up (hipGetSymbolAddress); make that
  *     call outside graph capture.

@@ -599,13 +599,14 @@ bool streaming_takes(size_t m, size_t n, size_t k, int lc, int la, int lb)
 } // namespace
 
 launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int la, int lb, size_t batch,
-                        size_t cus)
+                        size_t cus, bool any_rows)
 {
     const int   group = type_group_of(type_idx);
     launch_plan plan;
     // the table was tuned on single GEMMs: a batch changes how many tiles there are to
     // spread, which is the model's business
-    if(batch > 1 && model_plan_any_rows(m, n, k, lc, la, lb, &plan, batch, cus))
+    const auto estimate = any_rows ? &model_plan_any_rows : &model_plan;
+    if(batch > 1 && estimate(m, n, k, lc, la, lb, &plan, batch, cus))
     {
         return plan;
     }
@@ -632,10 +633,10 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     // ... then the model, and the nearest tuned entry for the rest.  (Not for a batch: the model
     // has declined it above, and one entry priced as if it had the chip to itself would have its K
     // cut for nothing: 128 x 511 x 511 x 4001 in 8 slices, 2048 tiles before any cut.)
-    if(batch == 1 && model_plan_any_rows(m, n, k, lc, la, lb, &plan, 1, cus))
+    if(batch == 1 && estimate(m, n, k, lc, la, lb, &plan, 1, cus))
     {
         launch_plan nearest;
-        if((m % 8 != 0 || n % 8 != 0 || k % 8 != 0)
+        if(any_rows && (m % 8 != 0 || n % 8 != 0 || k % 8 != 0)
            && (find_closest(tuned_table, tuned_count, m, n, k, group, la, lb, lc, &nearest)
                || (group != 0 && find_closest(tuned_table, tuned_count, m, n, k, 0, la, lb, lc, &nearest))))
         {

@@ -175,8 +175,11 @@ inline int type_group_of(int type_idx)
     return (type_idx == 1 || type_idx == 3) ? 1 : 0;
 }
 
+// any_rows: extents whose rows do not start on 16 bytes go to the estimate too.  Its plans for them copy
+// operands and cut K where the tables' entries do without; false is for a call that has no memory
+// for that.
 launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int la, int lb, size_t batch = 1,
-                        size_t cus = 0);
+                        size_t cus = 0, bool any_rows = true);
 
 } // namespace host
 } // namespace rocm_wmma_gemm

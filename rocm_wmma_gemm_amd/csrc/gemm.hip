@@ -587,9 +587,12 @@ int launch_streaming(int type_idx, const launch_plan& plan, const kernel_problem
     return 0;
 }
 
+// `last`: no other plan is to be tried where the scratch memory of this one cannot be had; the plan is then run
+// in a form that needs none (the caller's own scratch excepted, see below).  Otherwise
+// ROCM_WMMA_GEMM_ERR_SCRATCH, with nothing enqueued.
 template<class OutT>
 int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hipStream_t stream,
-           const fixed_scratch* fixed)
+           const fixed_scratch* fixed, bool last)
 {
     launch_plan plan = plan_in;
     if(plan.variant < 0 || plan.variant >= variant_total())
@@ -634,6 +637,7 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
     size_t      pack_bytes = 0;
     bool        packed     = false; // the kernel reads a padded copy of ...
     bool        copy_a = false, copy_b = false; // ... this operand
+    bool        dispensable = false; // the copies only just pay
     int         k_tail = 0; // columns of a partial last K tile that the kernel cuts off itself
 
     if(variant_at(plan.variant).pipeline != 0)
@@ -682,6 +686,9 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
                && pack_bytes <= workspace_limit_bytes / 2)
             {
                 packed   = true;
+                const operand_copies whole = padded_copies(p.M, p.N, p.K, p.a_kmajor, p.b_kmajor, a_rows, b_rows,
+                                                           dv.block_m, dv.block_n, dv.block_k, false);
+                dispensable = 2.0 * p.M * p.N * p.K < 256.0 * static_cast<double>(whole.elems_a + whole.elems_b);
                 k_tail   = edges ? static_cast<int>(p.K % dv.block_k) : 0;
                 lda      = copies.lda;
                 ldb      = copies.ldb;
@@ -807,13 +814,24 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
                                      ? 2 * stream_groups * v.block_m * v.block_n * sizeof(float)
                                      : (split_k > 1 ? plane_bytes * split_k * batches_per_launch : 0);
 
+    auto on_general_kernel = [&] {
+        launch_plan retry = plan;
+        retry.variant     = staged_fallback(v);
+        if(pick_mode(p, variant_at(retry.variant), retry.split_k) == static_cast<int>(device::load_mode::scalar))
+        {
+            retry.variant = 0;
+        }
+        return launch<OutT>(type_idx, retry, p, stream, fixed, true);
+    };
     char*           workspace = nullptr;
     workspace_lease lease; // held until the last kernel of this call is enqueued
     if(pack_bytes + partial_bytes > 0 && fixed != nullptr)
     {
         if(pack_bytes + partial_bytes > fixed->bytes)
         {
-            return ROCM_WMMA_GEMM_ERR_SCRATCH;
+            // (copies that only just pay are left out, beyond that the general kernel would be a
+            // surprise: 133 x 5000 x 3001 takes 278 us on it, 43 on copies)
+            return last && packed && dispensable ? on_general_kernel() : ROCM_WMMA_GEMM_ERR_SCRATCH;
         }
         workspace = fixed->ptr;
     }
@@ -822,17 +840,13 @@ int launch(int type_idx, const launch_plan& plan_in, const kernel_problem& p, hi
         workspace = lease.acquire(pack_bytes + partial_bytes, stream);
         if(workspace == nullptr)
         {
+            if(!last)
+            {
+                return ROCM_WMMA_GEMM_ERR_SCRATCH;
+            }
             if(packed)
             {
-                // no memory for the padded copies: take the general kernel instead
-                launch_plan retry = plan;
-                retry.variant     = staged_fallback(v);
-                if(pick_mode(p, variant_at(retry.variant), retry.split_k)
-                   == static_cast<int>(device::load_mode::scalar))
-                {
-                    retry.variant = 0;
-                }
-                return launch<OutT>(type_idx, retry, p, stream, fixed);
+                return on_general_kernel(); // no memory for the padded copies
             }
             split_k          = 1;
             tail_begin       = 0;
@@ -1038,43 +1052,52 @@ int run(int type_idx, const launch_plan* forced, void* C, void* A, void* B, size
         return 0;
     }
     const kernel_problem p = to_kernel_space(C, A, B, M, N, K, batch, layout_c, layout_a, layout_b);
-    launch_plan          plan
-        = forced ? *forced
-                 : select_plan(M, N, K, type_idx, layout_c, layout_a, layout_b, batch,
-                               compute_units_of_current_device());
-    if(!forced && variant_at(plan.variant).pipeline == 7 && !streaming_ok(p, variant_at(plan.variant)))
-    {
-        // the dispatcher prices shapes, not pointers: operands that the streaming kernel
-        // cannot take (base pointers or batch strides that are not 16-byte aligned) go
-        // to the general kernel with the shape heuristic's split
-        plan = heuristic_plan(M, N, K, layout_c);
-    }
-    if(variant_at(plan.variant).pipeline != 0
-       && lookup_kernel(type_idx, p.a_kmajor, p.b_kmajor, plan.variant,
-                        static_cast<int>(device::load_mode::vec_unguarded))
-              == nullptr)
-    {
-        // a tile that is not built for this pair of operand layouts (tile extents that
+    auto built = [&](const launch_plan& plan) {
+        // (a tile that is not built for this pair of operand layouts: tile extents that
         // are no multiple of 128 need that operand K-contiguous)
-        if(forced)
-        {
-            return -1;
-        }
-        plan.variant = staged_fallback(variant_at(plan.variant));
-    }
-    if(!forced && variant_at(plan.variant).pipeline == 0)
+        return variant_at(plan.variant).pipeline == 0
+               || lookup_kernel(type_idx, p.a_kmajor, p.b_kmajor, plan.variant,
+                                static_cast<int>(device::load_mode::vec_unguarded))
+                      != nullptr;
+    };
+    if(forced)
     {
+        return built(*forced) ? launch<OutT>(type_idx, *forced, p, stream, fixed, true) : -1;
+    }
+    const size_t cus    = compute_units_of_current_device();
+    auto         picked = [&](bool any_rows) {
+        launch_plan plan = select_plan(M, N, K, type_idx, layout_c, layout_a, layout_b, batch, cus, any_rows);
+        if(variant_at(plan.variant).pipeline == 7 && !streaming_ok(p, variant_at(plan.variant)))
+        {
+            // the dispatcher prices shapes, not pointers: operands that the streaming kernel
+            // cannot take (base pointers or batch strides that are not 16-byte aligned) go
+            // to the general kernel with the shape heuristic's split
+            plan = heuristic_plan(M, N, K, layout_c);
+        }
+        if(!built(plan))
+        {
+            plan.variant = staged_fallback(variant_at(plan.variant));
+        }
         // Same rule as in launch() for a staged variant picked directly: misaligned
         // operands go through the small tile.  A direct variant is left alone here:
         // launch() decides between padded copies and the staged kernels.
-        const variant_desc& v    = variant_at(plan.variant);
-        const int           mode = pick_mode(p, v, plan.split_k);
-        if(mode == static_cast<int>(device::load_mode::scalar) && !keeps_small_tile(p.M, p.N, p.batch, v.block_m, v.block_n, compute_units_of_current_device()))
+        const variant_desc& v = variant_at(plan.variant);
+        if(v.pipeline == 0 && pick_mode(p, v, plan.split_k) == static_cast<int>(device::load_mode::scalar)
+           && !keeps_small_tile(p.M, p.N, p.batch, v.block_m, v.block_n, cus))
         {
             plan.variant = 0;
         }
+        return plan;
+    };
+    const int rc = launch<OutT>(type_idx, picked(true), p, stream, fixed, false);
+    if(rc != ROCM_WMMA_GEMM_ERR_SCRATCH)
+    {
+        return rc;
     }
-    return launch<OutT>(type_idx, plan, p, stream, fixed);
+    // No memory for the plan (the caller's own scratch array is too small, or a capture forbids to
+    // allocate): for extents whose rows do not start on 16 bytes the tables' plan, which needs
+    // less or none, for all others the same plan once more, now in whatever form it can run.
+    return launch<OutT>(type_idx, picked(false), p, stream, fixed, true);
 }
 
 template<class T, class U>
