@@ -130,7 +130,7 @@ struct model_variant
     int block_m, block_n, block_k, waves_m, waves_n, pipeline;
 };
 #define RWG_VARIANT(IDX, BM, BN, BK, WM, WN, PIPE) {BM, BN, BK, WM, WN, PIPE},
-const model_variant model_variants[] = {
+constexpr model_variant model_variants[] = {
 #include "variants.def"
 };
 #undef RWG_VARIANT
@@ -168,6 +168,12 @@ double unaligned_copies_us(double bytes)
 
 // the general kernel's smallest square tile, 64 x 64 x 64
 constexpr int small_general_variant = 34;
+static_assert(model_variants[small_general_variant].pipeline == 0 && model_variants[small_general_variant].block_m == 64
+                  && model_variants[small_general_variant].block_n == 64,
+              "small_general_variant names the general kernel's 64 x 64 tile");
+static_assert(model_variants[0].pipeline == 0 && model_variants[0].block_m == 128 && model_variants[0].block_n == 128
+                  && model_variants[0].block_k == 32,
+              "variant 0 is the general kernel's 128 x 128 tile that unaligned operands go to");
 
 size_t ceil_div(size_t a, size_t b)
 {

@@ -109,44 +109,15 @@ struct gemm_args
                                // in that cache (16 x 8192 x 8192 20.6 us, 29 with the hint).
 };
 
-// What one workgroup works on.  Ids enumerate the whole tiles first, then (slice, split
-// tile) pairs, slices outermost.
-struct block_work
-{
-    int  tile_id; // position in the tile walk
-    int  slice, slices; // K slice of this workgroup and how many the tile has (1 = whole K)
-    bool walk_order; // tile_id counts along the walk already (see tile_of), else it is dealt by XCD
-};
-
-// Where every tile is split, the ids of the launch are renumbered as a whole, so that an XCD
-// owns a contiguous run of (slice, tile) pairs, a slice or two of K over all tiles.  Its L2 then
-// fetches its part of A and B once; with the tiles of every slice dealt over the XCDs,
-// as whole tiles are, each of the 8 L2s fetched nearly all of both operands, and the
-// fabric was the bound (704 x 896 x 12096 in 16 slices
-// 47.7 -> 44.5 us, 2048 x 1024 x 32768 in 8 145.7 -> 137.3, operands from HBM; a few slices of many
-// tiles gain nothing and lose nothing).
+// The work and the tile of workgroup b of a launch (tile_map.hpp).
 __device__ __forceinline__ block_work decode_block(const gemm_args& args, int b)
 {
-    if(b < args.tail_begin || args.k_slices == 1)
-    {
-        return {b, 0, 1, false};
-    }
-    const int split_tiles = args.grid_m * args.grid_n - args.tail_begin;
-    if(args.tail_begin == 0)
-    {
-        const int item  = xcd_remap(b, split_tiles * args.k_slices);
-        const int slice = item / split_tiles;
-        return {item - slice * split_tiles, slice, args.k_slices, true};
-    }
-    const int r     = b - args.tail_begin;
-    const int slice = r / split_tiles;
-    return {args.tail_begin + (r - slice * split_tiles), slice, args.k_slices, false};
+    return decode_block(b, args.grid_m * args.grid_n, args.tail_begin, args.k_slices);
 }
 
 __device__ __forceinline__ tile_coord tile_of(const gemm_args& args, const block_work& w)
 {
-    return banded_tile(w.walk_order ? w.tile_id : xcd_remap(w.tile_id, args.grid_m * args.grid_n), args.grid_m,
-                       args.grid_n, args.group);
+    return tile_of(w, args.grid_m, args.grid_n, args.group);
 }
 
 __device__ __forceinline__ block_work decode_block(const gemm_args& args)
@@ -319,8 +290,9 @@ struct operand_stage
                     // A chunk that the row holds whole is one 16-byte load at whatever
                     // address it starts on (an ordinary unaligned load to the compiler); only
                     // the chunk that K cuts goes element by element.  Eight loads of 2 bytes
-                    // for each bound the skinny shapes with an odd K (16 x 8192 x
-                    // 8191: 125 -> 61 us, with the tile that the dispatcher picks for them).
+                    // for each bound the skinny shapes with an odd K (same plan before and after, 16 x 8192 x
+                    // 8191: 124 -> 73 us on 128 x 128 tiles in 8 slices, 92 -> 60 on 64 x 64 in 6; 64 x 4096 x
+                    // 4095: 56 -> 31 in 15, 44 -> 22 in 12).
                     typedef u32x4 any_u32x4 __attribute__((aligned(2)));
                     if(row < rows_left && chunk * 8 + 8 <= k_left)
                     {

@@ -48,6 +48,46 @@ static int check_tilemap()
                 return fail("xcd_remap not a permutation");
         }
     }
+    // the workgroups of a launch: whole tiles once, split tiles once per slice, whatever is split
+    for(int gm : {1, 3, 8, 17})
+        for(int gn : {1, 2, 5, 16})
+            for(int group : {1, 4, -4})
+                for(int slices : {1, 2, 3, 8, 17})
+                    for(int tail : {0, 1, gm * gn / 2, gm * gn - 1})
+                    {
+                        const int tiles = gm * gn;
+                        if(slices == 1 && tail != 0)
+                            continue; // (a launch without slices has no split tail)
+                        const int total = tail + (tiles - tail) * slices;
+                        std::set<std::pair<std::pair<int, int>, int>> seen;
+                        for(int b = 0; b < total; ++b)
+                        {
+                            const block_work w = decode_block(b, tiles, tail, slices);
+                            const tile_coord t = tile_of(w, gm, gn, group);
+                            if(t.m < 0 || t.m >= gm || t.n < 0 || t.n >= gn || w.slice < 0 || w.slice >= w.slices)
+                                return fail("workgroup outside the launch's tiles and slices");
+                            if(!seen.insert({{t.m, t.n}, w.slice}).second)
+                                return fail("two workgroups on one slice of a tile");
+                            const tile_coord whole = map_tile(w.tile_id, gm, gn, group);
+                            if((b < tail || slices == 1) && (w.slices != 1 || t.m != whole.m || t.n != whole.n))
+                                return fail("whole tiles are not dealt as map_tile deals them");
+                            if(tail > 0 && b >= tail && (w.slices != slices || w.tile_id < tail || t.m != whole.m || t.n != whole.n))
+                                return fail("split tail is not where its reduce kernel looks for it");
+                        }
+                        if(static_cast<int>(seen.size()) != total)
+                            return fail("a slice of a tile without a workgroup");
+                        // every tile split: an XCD's workgroups are neighbours in the sequence of slices,
+                        // so that 8 XCDs over s slices touch at most s / 8 + 2 slices each
+                        if(tail == 0 && slices > 1)
+                            for(int xcd = 0; xcd < 8; ++xcd)
+                            {
+                                std::set<int> k;
+                                for(int b = xcd; b < total; b += 8)
+                                    k.insert(decode_block(b, tiles, tail, slices).slice);
+                                if(tiles >= 8 && static_cast<int>(k.size()) > slices / 8 + 2)
+                                    return fail("an XCD works on more slices of K than it has to");
+                            }
+                    }
     std::printf("tilemap ok\n");
     return 0;
 }

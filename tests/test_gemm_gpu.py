@@ -748,34 +748,45 @@ def test_partial_last_k_tile_on_the_persistent_kernel(loader):
 
 def test_rows_that_start_anywhere_on_the_persistent_kernel(loader):
     """Operands whose rows do not start on 16 bytes, which the one-wave-per-SIMD kernel reads
-    from copies padded along the row only, and C that it cannot store (odd extents, odd batch
-    strides, a C that starts one element late), which goes to another kernel.  What lies before
-    and behind C stays as it was."""
+    from copies padded along the row only, and C that it cannot store (odd extents in C's row, a C that
+    starts one element late), which goes to another kernel.  What lies before and behind C
+    stays as it was."""
     import torch
 
     solo = [v for v in loader.variants() if v.pipeline == 5]
-    cases = [  # M, N, K, batch, split field
-        (257, 511, 128, 1, 1),
+    cases = [  # M, N, K, batch, split field; a row of C is N long in the row-major layouts, M in the others
+        (257, 511, 128, 1, 1),     # no layout stores 16-byte pieces
         (304, 769, 200, 1, 1),     # K-contiguous rows aligned: no copies in A row / B column
         (255, 1001, 257, 1, 2),    # whole partial planes with odd rows, padded copies
         (259, 513, 264, 3, 1),     # odd batch stride of C
-        (513, 523, 648, 1, -1),    # walk by K tile: parts in slots of their own
-        (4353, 257, 64, 1, -2),    # more tiles than workgroups, the last wave split
+        (520, 523, 651, 1, -1),    # walk by K tile over copies (C column-major)
+        (4353, 4360, 137, 1, -2),  # more tiles than workgroups, the last wave split, copies
         (256, 512, 128, 1, 1),     # whole tiles, C one element late
-        (257, 520, 193, 1, 1),     # A row / B column: both copied, C in place
-        (259, 512, 1000, 3, 2),    # batch entries of an odd stride
+        (257, 520, 193, 3, 1),     # a batch on copies: strides of their own
+        (259, 512, 1001, 3, 2),    # batch entries of an odd stride, planes
+        (257, 520, 200, 1, 1),     # A column-major: its copy ends in the middle of a K tile
         (513, 528, 649, 1, -1),
+        (513, 523, 648, 1, -1),    # aligned rows, C odd either way: whole tiles elsewhere
+        (4353, 257, 64, 1, -2),    # fewer tiles than workgroups, one K step: nothing to split
+        (259, 512, 1000, 3, 2),    # a batch without copies, rows and planes ragged
     ]
+    stored = set()
     for i, v in enumerate(solo):
         for n, (M, N, K, batch, split) in enumerate(cases):
             tname = list(TYPE_PAIRS)[(n + i) % 4]
             din, dout = TYPE_PAIRS[tname]
-            for (lc, la, lb) in [l for l in [(0, 0, 1), (1, 1, 0), (0, 0, 0), (1, 1, 1)] if built_for(v, *l)]:
+            layouts = [(0, 0, 1), (1, 1, 0)] if N > 4000 else [(0, 0, 1), (1, 1, 0), (0, 0, 0), (1, 1, 1), (0, 1, 0)]
+            for (lc, la, lb) in [l for l in layouts if built_for(v, *l)]:
                 A = np.concatenate([O.init_matrix(M, K, la, din, seed=330 + b) for b in range(batch)])
                 B = np.concatenate([O.init_matrix(K, N, lb, din, seed=360 + b) for b in range(batch)])
-                size, before = M * N * batch, 9 if n % 2 == 0 and n < 7 else 8
+                size, before = M * N * batch, 9 if (M, N) in ((256, 512), (257, 511), (255, 1001)) else 8
                 buf = torch.full((size + 32,), float("nan"), dtype=torch_dtype(dout), device="cuda")
                 out = buf[before:before + size]
+                rows, cols = (M, N) if lc == 0 else (N, M)
+                if before == 8 and cols % 8 == 0 and (batch == 1 or M * N % 8 == 0):
+                    stored.add(n)  # (runs on the persistent kernel itself)
+                if split == -2 and N > 4000:
+                    assert -(-rows // v.block_m) * -(-cols // v.block_n) > 256
                 where = f"variant {v.index} {M}x{N}x{K} batch {batch} split {split} layouts C{lc} A{la} B{lb} {tname}"
                 rc = loader.run_variant(v.index, 4, split, out, to_device(A, din), to_device(B, din), M, N, K, lc, la,
                                         lb, batch_count=batch)
@@ -789,6 +800,33 @@ def test_rows_that_start_anywhere_on_the_persistent_kernel(loader):
                                              B[b * K * N:(b + 1) * K * N], M, N, K, lc, la, lb, din, dout)
                     except AssertionError as e:
                         raise AssertionError(f"{where} entry {b}: {e}") from None
+    assert stored == {1, 4, 5, 7, 8, 9, 10, 13}, stored
+
+
+@pytest.mark.parametrize("split", [2, 7, 8, 9, 16, 17])
+def test_whole_plane_reduce_at_the_edges_of_its_unroll(loader, split):
+    """The sum over partial planes, eight planes at a time with a remainder, four elements a thread where
+    planes and C allow it and one where they do not (odd planes, a batch of them, a C that starts
+    one element late)."""
+    import torch
+
+    v = loader.variants()[34]  # 64 x 64 x 64 tiles: any shape, K steps of 64
+    K = 64 * split
+    for n, (M, N, batch, late) in enumerate([(64, 68, 1, 0), (63, 65, 1, 0), (62, 66, 2, 0), (61, 63, 3, 0), (64, 64, 2, 1)]):
+        din, dout = TYPE_PAIRS[list(TYPE_PAIRS)[n % 4]]
+        A = np.concatenate([O.init_matrix(M, K, 0, din, seed=510 + b) for b in range(batch)])
+        B = np.concatenate([O.init_matrix(K, N, 1, din, seed=540 + b) for b in range(batch)])
+        size = M * N * batch
+        buf = torch.full((size + 16,), float("nan"), dtype=torch_dtype(dout), device="cuda")
+        out = buf[8 + late:8 + late + size]
+        assert loader.run_variant(v.index, 4, split, out, to_device(A, din), to_device(B, din), M, N, K, 0, 0, 1,
+                                  batch_count=batch) == 0
+        torch.cuda.synchronize()
+        assert torch.isnan(buf[:8 + late]).all() and torch.isnan(buf[8 + late + size:]).all(), (M, N, batch)
+        gpu = to_host(out.contiguous(), dout)
+        for b in range(batch):
+            check_against_oracle(gpu[b * M * N:(b + 1) * M * N], A[b * M * K:(b + 1) * M * K],
+                                 B[b * K * N:(b + 1) * K * N], M, N, K, 0, 0, 1, din, dout)
 
 
 @pytest.mark.parametrize("M,N,K,batch,type_name,layouts,route", [
