@@ -216,7 +216,7 @@ operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b
 // On the 208 tuned entries the model can serve, its pick is on average 2.7 % slower than
 // the tuner's, 25 % at worst.
 //
-// `any_rows`: also for extents whose rows do not start on 16 bytes (see model_plan_any_rows).
+// `any_rows`: also for extents that are no multiples of 8 (see model_plan_any_rows).
 namespace
 {
 bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch,
@@ -245,7 +245,8 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     const bool   regular = rows % 8 == 0 && cols % 8 == 0 && a_rows && b_rows;
     // (a C that cannot take 16-byte pieces is not the persistent kernel's.  Where that or a copy
     // comes in and 256 x 256 tiles cover half the chip, the nearest tuned entry's large tile serves
-    // as well or better: 3000 x 3000 x 3001, all row-major, 79 us against 89.  Counted for one entry
+    // as well or better: 3000 x 3000 x 3001, all row-major, 79 us against 89; of 247 drawn shapes beyond the line
+    // 63 would be more than 5 % slower by the estimate, of 283 below it 7.  Counted for one entry
     // of a batch: what the table would give 64 x 856 x 673 x 1014 is a small tile in 4 slices, 544 us,
     // the estimate 243)
     const bool   pieces  = cols % 8 == 0;
@@ -442,10 +443,10 @@ bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_pla
     return estimated_plan(m, n, k, lc, la, lb, out, batch, cus_of_device, false);
 }
 
-// Any number of tokens against a weight (133 x 5560 x 10232), odd extents: the nearest tuned
-// entry knows neither how many tiles there are nor that a small operand is cheap to copy
-// (133 x 5560 x 10232
-// 134 -> 90 us, 250 x 1001 x 40001 814 -> 75, 2001 x 2001 x 16384 321 -> 185).  Same arithmetic, with the copies of the operands that need them priced in.
+// Any number of tokens against a weight, odd extents: the nearest tuned
+// entry knows neither how many tiles there are nor that a small operand is cheap to copy.  Same
+// arithmetic, with the copies priced in (133 x 5560 x 10232 134 -> 90 us, 250 x 1001 x 40001 814 -> 75,
+// 2001 x 2001 x 16384 321 -> 185; over 1000 drawn shapes 0.73 of the entries' time).
 bool model_plan_any_rows(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch,
                          size_t cus_of_device)
 {

@@ -1,7 +1,7 @@
 // Shape -> launch plan.  The tuned table comes from gemm_config_gfx950_*.json via
 // config/generate_config.py; shapes the table does not name are served by a time
-// estimate over the compiled variants when they are regular (select_plan: K a multiple
-// of 64, extents multiples of 8), else by the table's nearest entry, and layouts the
+// estimate over the compiled variants (select_plan says which), skinny ones with unaligned rows by
+// the general kernel, the rest by the table's nearest entry, and layouts the
 // table does not cover at all by a shape heuristic.
 //
 // select_plan_from follows the reference's generated find_best_config /
@@ -153,12 +153,14 @@ operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b
 bool keeps_small_tile(size_t m, size_t n, size_t batch, int block_m, int block_n, size_t cus);
 
 // Estimated-time choice among the compiled variants for a shape without a tuned entry;
-// false for shapes it does not cover (ragged K, odd extents).
+// false for shapes it does not cover: extents that are no multiples of 8, unless they stream, and
+// K-contiguous rows that do not start on 16 bytes.
 // cus: compute units of the GPU the plan is for (0: the GPU the constants were measured on).
 bool model_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch = 1,
                 size_t cus = 0);
-// The same, also for extents whose rows do not start on 16 bytes (an odd number of tokens,
-// odd features): the operands that need it are copied first.
+// The same for the shapes above, and also for other extents (an odd number of tokens, odd
+// features), operands copied first where a kernel needs that; false where the nearest tuned entry
+// serves as well.
 bool model_plan_any_rows(size_t m, size_t n, size_t k, int lc, int la, int lb, launch_plan* out, size_t batch = 1,
                          size_t cus = 0);
 // The streaming kernel's plans alone (skinny shapes: one extent at most 128, or small ones:

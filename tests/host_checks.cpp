@@ -398,6 +398,16 @@ static int check_select()
         return fail("model: a tail wave whose slices need two passes stays whole");
     if(!model_plan(4096, 4096, 1000, 0, 0, 1, &p) || tiles[p.variant].pipeline != 5)
         return fail("model: ragged K with aligned rows belongs to the persistent kernel");
+    // the function that dispatch asks is the one held to the recorded sweep: the same plan for regular extents
+    for(size_t m : {16, 64, 128, 304, 1024, 4352})
+        for(size_t k : {256, 1000, 4096, 20480})
+            for(int l = 0; l < 8; ++l)
+            {
+                launch_plan a, b;
+                const bool  fa = model_plan(m, 2048, k, l & 1, (l >> 1) & 1, l >> 2, &a), fb = model_plan_any_rows(m, 2048, k, l & 1, (l >> 1) & 1, l >> 2, &b);
+                if(fa != fb || (fa && (a.variant != b.variant || a.swizzle != b.swizzle || a.split_k != b.split_k || a.touch != b.touch)))
+                    return fail("model: regular extents by either function");
+            }
     // K-contiguous rows that are not 16-byte aligned, odd extents: not its business ...
     if(model_plan(4096, 4096, 1001, 0, 0, 1, &p) || model_plan(4095, 4096, 4096, 0, 0, 1, &p))
         return fail("model must leave irregular shapes alone");
