@@ -5,6 +5,7 @@
 
 #include <initializer_list>
 #include <limits>
+#include <vector>
 
 #include "config_generated.hpp"
 
@@ -29,11 +30,44 @@ bool same_slot(const tuned_entry& e, int type_group, int la, int lb, int lc)
 {
     return e.type_group == type_group && e.layout_a == la && e.layout_b == lb && e.layout_c == lc;
 }
+
+// The tuned table by type group and layouts, in the table's order.  A call looks up to six times for
+// an entry, each time in one of the 16 slots: with the whole table of 1376 entries walked every time the look-ups
+// of a call that ends at the nearest entry took 2 us of host time, which small problems show.
+struct tuned_slots
+{
+    std::vector<tuned_entry> slot[16];
+    tuned_slots()
+    {
+        for(size_t i = 0; i < generated::entry_count; ++i)
+        {
+            const tuned_entry& e = generated::entries[i];
+            slot[index(e.type_group, e.layout_a, e.layout_b, e.layout_c)].push_back(e);
+        }
+    }
+    static int index(int type_group, int la, int lb, int lc)
+    {
+        return ((type_group & 1) << 3) | ((la & 1) << 2) | ((lb & 1) << 1) | (lc & 1);
+    }
+};
+
+// The part of a table that a look-up has to see: its slot of the tuned table, all of any other.
+void narrow(const tuned_entry*& table, size_t& count, int type_group, int la, int lb, int lc)
+{
+    if(table == tuned_table && count == tuned_count)
+    {
+        static const tuned_slots         slots;
+        const std::vector<tuned_entry>& s = slots.slot[tuned_slots::index(type_group, la, lb, lc)];
+        table                            = s.data();
+        count                            = s.size();
+    }
+}
 } // namespace
 
 bool find_exact(const tuned_entry* table, size_t count, size_t m, size_t n, size_t k,
                 int type_group, int la, int lb, int lc, launch_plan* out)
 {
+    narrow(table, count, type_group, la, lb, lc);
     for(size_t i = 0; i < count; ++i)
     {
         const tuned_entry& e = table[i];
@@ -49,6 +83,7 @@ bool find_exact(const tuned_entry* table, size_t count, size_t m, size_t n, size
 bool find_closest(const tuned_entry* table, size_t count, size_t m, size_t n, size_t k,
                   int type_group, int la, int lb, int lc, launch_plan* out)
 {
+    narrow(table, count, type_group, la, lb, lc);
     bool   any       = false;
     size_t best_kgap = std::numeric_limits<size_t>::max();
     size_t best_k    = 0;
@@ -202,7 +237,10 @@ operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b
     c.elems_a = !c.a ? 0 : c.lda * (!edges ? (a_kmajor ? m_pad : k_pad) : a_kmajor ? m : k);
     c.elems_b = !c.b ? 0 : c.ldb * (!edges ? (b_kmajor ? n_pad : k_pad) : b_kmajor ? n : k);
     const double copied = static_cast<double>(c.elems_a + c.elems_b);
-    c.pays              = copied > 0.0 && k >= 128 && 2.0 * m * n * k >= copy_pays_flops * copied;
+    const double flops  = 2.0 * m * n * k;
+    c.pays              = copied > 0.0
+             && ((k >= 128 && flops >= copy_pays_flops_aligned * copied)
+                 || (k >= 256 && flops >= copy_pays_flops * copied && !(a_rows && b_rows)));
     return c;
 }
 
@@ -319,15 +357,12 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
         const operand_copies copies    = padded_copies(rows, cols, k, a_kmajor, b_kmajor, a_rows, b_rows, bm, bn, 64, v.pipeline == 5);
         if(copies.a || copies.b)
         {
-            const double elems = static_cast<double>(copies.elems_a + copies.elems_b);
-            if(regular ? 2.0 * rows * cols * k < copy_pays_flops * elems : !copies.pays)
+            if(!copies.pays || k < 256)
             {
-                continue; // (the launch takes the general kernel instead)
+                continue; // (see above; the launch takes the general kernel where they do not pay)
             }
-            // (regular extents are priced as in the fit of the constants.  Below a K of 128 nothing is
-            // copied for them and the launch takes the general kernel's tile of the same size: 128 x 576 x 64
-            // 8.1 us, 8.5 by the nearest entry)
-            const double bytes = elems * static_cast<double>(batch) * 4.0;
+            // (regular extents are priced as in the fit of the constants)
+            const double bytes = static_cast<double>(copies.elems_a + copies.elems_b) * static_cast<double>(batch) * 4.0;
             copies_us          = regular ? launch_us + bytes / model_measured.copy_bytes_per_us : unaligned_copies_us(bytes);
         }
         auto consider = [&](double t, int split) {
@@ -417,6 +452,19 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     const bool   compete = skinny <= 64 || (skinny <= 128 && one_pass)
                          || (rows * cols <= (size_t{1} << 20) && k <= 4096)
                          || (!regular && skinny <= 128 && best_copies_large);
+    // Regular, and no tile without copies that are too dear for it: less than 192 rows or columns that are no
+    // multiple of 128.  Where the streaming plan does not run in one pass either, or needs a longer K, the
+    // general kernel's 64 x 64 tile reads them as they are (128 x 704 x 192 3.4 us, 13.2 on copies and 6.8 on
+    // its 128 x 128 tile; 67 x 160 x 200 x 256 8.3 us, 22.3 streamed, 11.4; in one pass 48 x 256 x 512 6.0 and
+    // 4.3 streamed).
+    if(!found && regular && (!have_stream || (!one_pass && k <= 768)))
+    {
+        out->variant = small_general_variant;
+        out->swizzle = 4;
+        out->split_k = 1;
+        out->touch   = 0;
+        return true;
+    }
     // (no tiled plan moves A and B faster than operand_bytes_per_us, which is what bounds the
     // skinny shapes; the estimates above rank the tiled plans among themselves without it)
     const double tiled_us = std::max(best, launch_us + operand_us);
@@ -643,7 +691,10 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     if(batch == 1 && estimate(m, n, k, lc, la, lb, &plan, 1, cus))
     {
         launch_plan nearest;
-        if(any_rows && (m % 8 != 0 || n % 8 != 0 || k % 8 != 0)
+        const int    pipeline = model_variants[plan.variant].pipeline;
+        const size_t elements = m * n;
+        const bool   short_sum = pipeline != 7 && std::min(m, n) > 128 && elements > (size_t{1} << 20) && elements <= (size_t{1} << 21) && k <= 2048;
+        if(any_rows && (pipeline == 5 || short_sum) && (m % 8 != 0 || n % 8 != 0 || k % 8 != 0)
            && (find_closest(tuned_table, tuned_count, m, n, k, group, la, lb, lc, &nearest)
                || (group != 0 && find_closest(tuned_table, tuned_count, m, n, k, 0, la, lb, lc, &nearest))))
         {
@@ -653,11 +704,8 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
             // streaming, 18 us and 25 by the estimate, 774 x 2104 x 1104 22 and 26; 1544 x 900 x 608, general, 12
             // and 18, 290 x 4416 x 1792 29 and 37).  Not further: 269 x 4808 x 3816 50 us and 39,
             // 2657 x 1344 x 1088 39 and 24.
-            const size_t elements = m * n;
-            if((model_variants[nearest.variant].pipeline == 7 || model_variants[nearest.variant].pipeline == 0)
-               && model_variants[plan.variant].pipeline != 7 && nearest.split_k <= 1 && std::min(m, n) > 128
-               && elements > (size_t{1} << 20) && elements <= (size_t{1} << 21) && k <= 2048
-               && streaming_takes(m, n, k, lc, la, lb))
+            if(short_sum && (model_variants[nearest.variant].pipeline == 7 || model_variants[nearest.variant].pipeline == 0)
+               && nearest.split_k <= 1 && streaming_takes(m, n, k, lc, la, lb))
             {
                 return nearest;
             }
