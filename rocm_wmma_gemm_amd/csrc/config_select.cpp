@@ -729,7 +729,12 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
     // for a handful of rows.  The general kernel's small tiles, K cut until there are enough
     // workgroups, all of them at once: three of 64 x 64 to a compute unit (8 x 3678 x 3817, odd K: 41.2 us
     // on the 128 x 128 tile with 15 slices, 28.0 on this one with 12), two of 128 x 128.
-    // Up to 64 rows the 64 x 64 tile.  From 65 on it takes two rows of tiles, each of which reads all of
+    // Up to 64 rows the 64 x 64 tile, unless the general kernel has to read element by element throughout:
+    // no operand K-contiguous and a K of 1024 (72 shapes, against the entries: 128 x 128 tiles 0.83, 64 x 64
+    // 1.04; below, 1242 x 23 x 304 15 us and 12), or a handful of rows against 30 MB and more that are not (8 x 7570 x 2936 30 us and 40, 4 x 2132 x 8269
+    // 31 and 35; below, 10 x 1330 x 1786 25 and 15; more rows, 37 x 5133 x 4395 41 and 41, 64 x 6012 x 14831 102
+    // and 88; beyond 16384 columns, where two tiles a compute unit are few, 7 x 24345 x 6771 228 and 221).
+    // From 65 on it takes two rows of tiles, each of which reads all of
     // the large operand, and the 128 x 128 tile is ahead where it covers the GPU: by its tiles
     // alone (from one to two compute units on: 104 x 986 x 207 x 64 20.8 us, 39.2 on 64 x 64), or cut along a K
     // of 2048 and more (80 x 8192 x 8191, B row-major 76 us against 124; 112 x 16000 x 3003 73 and 67;
@@ -744,8 +749,14 @@ launch_plan select_plan(size_t m, size_t n, size_t k, int type_idx, int lc, int 
         const size_t small = ceil_div(m, size_t{64}) * ceil_div(n, size_t{64}) * batch;
         const size_t large = ceil_div(m, size_t{128}) * ceil_div(n, size_t{128}) * batch;
         const size_t cut   = std::max<size_t>(1, std::min({2 * units / large, k / 256, size_t{64}})); // 8 K steps of 32 a slice
-        const bool   once  = la == 0 && lb == 1 && batch == 1 && std::max(m, n) * k < (size_t{1} << 25);
-        const bool   wide  = std::min(m, n) > 64 && !once && (large * 2 >= units || (k >= 2048 && large * cut >= units));
+        const size_t skinny = std::min(m, n), weight = std::max(m, n) * k; // (elements of the large operand)
+        const bool   a_k = la == 0, b_k = lb == 1; // K-contiguous, whatever the layout of C
+        const bool   large_k = n >= m ? b_k : a_k;
+        const bool   once   = a_k && b_k && batch == 1 && weight < (size_t{1} << 25);
+        const bool   wide   = skinny > 64    ? !once && (large * 2 >= units || (k >= 2048 && large * cut >= units))
+                              : batch > 1    ? false
+                              : !a_k && !b_k ? k >= 1024
+                                             : !large_k && skinny <= 24 && weight >= 15000000 && std::max(m, n) <= 16384;
         plan.variant       = wide ? 0 : small_general_variant;
         plan.swizzle       = 4;
         plan.touch         = 0;

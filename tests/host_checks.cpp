@@ -303,6 +303,15 @@ static int check_select()
             if(r.variant != q.variant || r.split_k != q.split_k)
                 return fail("select: skinny N like skinny M");
         }
+        // up to 64 rows: 128 x 128 tiles where everything is read element by element
+        const struct { size_t m, n, k; int la, lb, bm; } few[] = {{7, 7571, 2937, 0, 0, 128}, {7, 1331, 1787, 0, 0, 64}, {37, 7571, 2937, 0, 0, 64},
+            {7, 24345, 6771, 0, 0, 64}, {7, 7571, 2937, 0, 1, 64}, {7, 1331, 1787, 1, 0, 128}, {50, 7571, 2937, 1, 0, 128}, {50, 7571, 1001, 1, 0, 64}, {7, 7571, 2937, 1, 1, 64}};
+        for(const auto& x : few)
+        {
+            const launch_plan q = select_plan(x.m, x.n, x.k, 0, 0, x.la, x.lb), r = select_plan(x.n, x.m, x.k, 0, 1, 1 - x.lb, 1 - x.la);
+            if(tiles[q.variant].pipeline != 0 || tiles[q.variant].bm != x.bm || r.variant != q.variant || r.split_k != q.split_k)
+                return fail("select: a few unaligned rows");
+        }
         // both operands K-contiguous: 128 x 128 tiles from 64 MB of the large operand on
         if(tiles[select_plan(80, 8192, 4095, 0, 0, 0, 1).variant].bm != 64 || tiles[select_plan(80, 8193, 4097, 0, 0, 0, 1).variant].bm != 128)
             return fail("select: skinny shape with unaligned K-contiguous rows");
