@@ -472,10 +472,11 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     // plan takes 1.6 times its estimate, the tiled ones less than theirs, and the two are level
     // where the estimates are 1 to 2.  391 timed pairs with one workgroup to a streaming tile: 0.86 of
     // the tiled time beyond that ratio, 171 x 1088 x 4800 14 us and 25, 141 x 5440 x 7744 44 and 69; 1.22 below
-    // it.  Not for its 16-wide tiles, 1.15, nor past a K of 8192: 189 x 2048 x 14120 65 us, 54 tiled)
-    const bool stream_late = !regular && skinny > 128 && k > 4096 && k <= 8192 && have_stream && stream_best.split_k == 1
+    // it.  Past a K of 8192 they are level at 1 to 2.5, 0.84 beyond (182 x 4288 x 11712 61 us and 84).  Not for its
+    // 16-wide tiles, 1.15)
+    const bool stream_late = !regular && skinny > 128 && k > 4096 && have_stream && stream_best.split_k == 1
                              && model_variants[stream_best.variant].block_m > 16 && model_variants[stream_best.variant].block_n > 16
-                             && 2.0 * stream_us < tiled_us;
+                             && (k <= 8192 ? 2.0 : 2.5) * stream_us < tiled_us;
     if(have_stream && (!found || stream_late || (stream_us < tiled_us && compete)))
     {
         *out  = stream_best;
