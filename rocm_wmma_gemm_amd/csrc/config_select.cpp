@@ -353,14 +353,21 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
         const double tile_bytes = static_cast<double>(bm * bn) * 4.0;
         // only the persistent kernel takes ragged M, N or K as they are; the others run on
         // padded copies of the operands that need them (one more launch)
-        double               copies_us = 0.0;
-        const operand_copies copies    = padded_copies(rows, cols, k, a_kmajor, b_kmajor, a_rows, b_rows, bm, bn, 64, v.pipeline == 5);
-        if(copies.a || copies.b)
+        double     copies_us    = 0.0;
+        bool       large_copied = false; // the larger operand is
+        const bool whole        = v.pipeline == 5 || (tm * bm == rows && tn * bn == cols && kt * 64 == k);
+        if(!(rows_ok && whole))
         {
-            if(!copies.pays || k < 256)
+            if(k < 256)
             {
-                continue; // (see above; the launch takes the general kernel where they do not pay)
+                continue; // (see above)
             }
+            const operand_copies copies = padded_copies(rows, cols, k, a_kmajor, b_kmajor, a_rows, b_rows, bm, bn, 64, v.pipeline == 5);
+            if(!copies.pays)
+            {
+                continue; // (the launch takes the general kernel where they do not pay)
+            }
+            large_copied = cols >= rows ? copies.b : copies.a;
             // (regular extents are priced as in the fit of the constants)
             const double bytes = static_cast<double>(copies.elems_a + copies.elems_b) * static_cast<double>(batch) * 4.0;
             copies_us          = regular ? launch_us + bytes / model_measured.copy_bytes_per_us : unaligned_copies_us(bytes);
@@ -371,7 +378,7 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
             {
                 found        = true;
                 best         = t;
-                best_copies_large = cols >= rows ? copies.b : copies.a;
+                best_copies_large = large_copied;
                 out->variant = i;
                 out->swizzle = 4;
                 out->split_k = split;
