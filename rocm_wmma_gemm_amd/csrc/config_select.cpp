@@ -479,11 +479,12 @@ bool estimated_plan(size_t m, size_t n, size_t k, int lc, int la, int lb, launch
     // plan takes 1.6 times its estimate, the tiled ones less than theirs, and the two are level
     // where the estimates are 1 to 2.  391 timed pairs with one workgroup to a streaming tile: 0.86 of
     // the tiled time beyond that ratio, 171 x 1088 x 4800 14 us and 25, 141 x 5440 x 7744 44 and 69; 1.22 below
-    // it.  Past a K of 8192 they are level at 1 to 2.5, 0.84 beyond (182 x 4288 x 11712 61 us and 84).  Not for its
-    // 16-wide tiles, 1.15)
+    // it.  Past a K of 8192 they are level at 1 to 2.5 and only the 64 x 64 tile is worth it, 0.78 of the tiled time
+    // beyond (182 x 4288 x 11712 61 us and 84); 32 x 64 gains nothing there, 133 x 5560 x 10232 133 and 89.  Nor do the
+    // 16-wide tiles anywhere, 1.15)
+    const int  stream_side = !have_stream ? 0 : std::min(model_variants[stream_best.variant].block_m, model_variants[stream_best.variant].block_n);
     const bool stream_late = !regular && skinny > 128 && k > 4096 && have_stream && stream_best.split_k == 1
-                             && model_variants[stream_best.variant].block_m > 16 && model_variants[stream_best.variant].block_n > 16
-                             && (k <= 8192 ? 2.0 : 2.5) * stream_us < tiled_us;
+                             && (k <= 8192 ? stream_side > 16 && 2.0 * stream_us < tiled_us : stream_side >= 64 && 2.5 * stream_us < tiled_us);
     if(have_stream && (!found || stream_late || (stream_us < tiled_us && compete)))
     {
         *out  = stream_best;
