@@ -240,7 +240,8 @@ operand_copies padded_copies(size_t m, size_t n, size_t k, bool a_kmajor, bool b
     const double flops  = 2.0 * m * n * k;
     c.pays              = copied > 0.0
              && ((k >= 128 && flops >= copy_pays_flops_aligned * copied)
-                 || (k >= 256 && flops >= copy_pays_flops * copied && !(a_rows && b_rows)));
+                 || (flops >= copy_pays_flops * copied
+                     && (a_rows && b_rows ? k >= 2048 && std::max(m, n) >= 5120 : k >= 256)));
     return c;
 }
 

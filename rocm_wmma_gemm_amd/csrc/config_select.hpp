@@ -123,11 +123,13 @@ bool find_exact(const tuned_entry* table, size_t count, size_t m, size_t n, size
 bool find_closest(const tuned_entry* table, size_t count, size_t m, size_t n, size_t k,
                   int type_group, int la, int lb, int lc, launch_plan* out);
 launch_plan heuristic_plan(size_t m, size_t n, size_t k, int lc);
-// Operations per element copied from which on padded copies pay against the general kernel.  Operands whose
-// rows are aligned, which it reads 16 bytes at a time: 256 (832 x 128 x 128, 238 of them, 12.4 us copied,
-// 6.0 by the general kernel's 128 x 128 tile).  Unaligned rows: 200, about 100 rows against an
-// odd weight, from a K of 256 on (64 x 4096 x 4095: 32.8 us copied, 20.5 by the general kernel; 96 rows 33.7
-// and 27.4; 133 x 5000 x 3001 43.1 and 278; 441 x 806 x 150 13.4 and 9.9).
+// Operations per element copied from which on padded copies pay against the general kernel: 256, and
+// 200 where its way of loading costs more.  Unaligned rows, which it reads a few bytes at a time, from a K of
+// 256 on: about 100 rows against an odd weight (64 x 4096 x 4095: 32.8 us copied, 20.5 by the general kernel; 96
+// rows 33.7 and 27.4; 133 x 5000 x 3001 43.1 and 278; 441 x 806 x 150 13.4 and 9.9).  Aligned rows from a K
+// of 2048 and 5120 columns on (133 x 5560 x 10232, 251 of them, 89 us copied, 133 by the next best plan, 131 x
+// 11920 x 2696 0.64 of its time; with fewer columns, 133 x 1088 x 4672 26 and 17; 832 x 128 x 128, 238 of them, 12.4
+// copied and 6.0 by the general kernel's 128 x 128 tile).
 constexpr double copy_pays_flops_aligned = 256.0, copy_pays_flops = 200.0;
 
 // The padded copies that a direct-to-LDS tile needs of the operands of one problem, in kernel
